@@ -17,7 +17,7 @@ enum class ElemType { F32, F16, BF16 };
 // Contiguous causal GQA attention (the reference's self_attention op).
 // Small grids (few query rows x heads) split the keys over workgroups into
 // fp32 partials in `workspace` (selfAttentionWorkspaceBytes; 0: none needed).
-size_t selfAttentionWorkspaceBytes(int L, int S, int nh, int dv);
+size_t selfAttentionWorkspaceBytes(ElemType type, int L, int S, int nh, int nkvh, int d, int dv, float scale);
 void selfAttention(void *out, const void *q, const void *k, const void *v, ElemType type, int L, int S, int nh,
                    int nkvh, int d, int dv, float scale, void *stream, void *workspace);
 

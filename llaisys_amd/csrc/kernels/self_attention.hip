@@ -18,6 +18,7 @@
 // Online softmax in base 2 per wave, fp32 throughout; the waves' states
 // (m, l, o) meet in LDS and one rounding to the output type ends it.
 #include "launch.hpp"
+#include "self_attention.hpp"
 
 #include "../device/hip_check.hpp"
 
@@ -25,6 +26,8 @@
 #include <hip/hip_fp16.h>
 
 #include <algorithm>
+#include <mutex>
+#include <vector>
 
 namespace llaisys::kernels {
 
@@ -213,7 +216,7 @@ __global__ void __launch_bounds__(64 * kWaves) selfAttentionKernel(T *__restrict
     }
 }
 
-constexpr int kSplitGrid = 1024, kMaxSplits = 16;
+constexpr int kSplitGrid = 1024, kMaxSplits = kSelfAttentionMaxSplits;
 
 // Merge the NS key splits of (query i, head h): weights 2^(m_z - M); one
 // thread per output dim (dv <= 256).
@@ -255,6 +258,24 @@ int splitsFor(int L, int S, int nh) {
     return int(std::max<long>(1, std::min<long>({long(chunks), long(kMaxSplits), kSplitGrid / base})));
 }
 
+int computeUnits() {
+    static std::mutex mu;
+    static std::vector<int> cache;
+    int dev = 0;
+    HIP_CHECK(hipGetDevice(&dev));
+    std::lock_guard<std::mutex> lock(mu);
+    if (size_t(dev) >= cache.size()) cache.resize(dev + 1, 0);
+    if (!cache[dev]) HIP_CHECK(hipDeviceGetAttribute(&cache[dev], hipDeviceAttributeMultiprocessorCount, dev));
+    return cache[dev];
+}
+
+template <typename T>
+void merge(void *out, const float *part, int L, int nh, int dv, int ns, hipStream_t stream) {
+    hipLaunchKernelGGL(selfAttentionMergeKernel<T>, dim3(L, nh), dim3(dv > 128 ? 256 : 128), 0, stream,
+                       static_cast<T *>(out), part, nh, dv, ns);
+    HIP_CHECK(hipGetLastError());
+}
+
 template <typename T>
 void launch(void *out, const void *q, const void *k, const void *v, int L, int S, int nh, int nkvh, int d, int dv,
             float scale, hipStream_t stream, float *part) {
@@ -280,18 +301,17 @@ void launch(void *out, const void *q, const void *k, const void *v, int L, int S
         hipLaunchKernelGGL((selfAttentionKernel<T, false, false>), grid, block, 0, stream, o, qq, kk, vv, L, S, nh,
                            nkvh, d, dv, scale_log2, part);
     HIP_CHECK(hipGetLastError());
-    if (ns > 1) {
-        hipLaunchKernelGGL(selfAttentionMergeKernel<T>, dim3(L, nh), dim3(dv > 128 ? 256 : 128), 0, stream, o, part,
-                           nh, dv, ns);
-        HIP_CHECK(hipGetLastError());
-    }
+    if (ns > 1) merge<T>(out, part, L, nh, dv, ns, stream);
 }
 
 } // namespace
 
-size_t selfAttentionWorkspaceBytes(int L, int S, int nh, int dv) {
+size_t selfAttentionWorkspaceBytes(ElemType type, int L, int S, int nh, int nkvh, int d, int dv, float scale) {
     if (L <= 0 || nh <= 0) return 0;
-    const int ns = splitsFor(L, S, nh);
+    // (Operands that are not 16 B aligned take the general kernel.)
+    int ns = splitsFor(L, S, nh);
+    if (selfAttentionMfmaTakes(type, L, S, nkvh, d, dv, scale))
+        ns = std::max(ns, planSelfAttentionMfma(type, L, S, nh, nkvh, computeUnits()).splits);
     return ns > 1 ? size_t(L) * nh * ns * (dv + 2) * sizeof(float) : 0;
 }
 
@@ -301,6 +321,21 @@ void selfAttention(void *out, const void *q, const void *k, const void *v, ElemT
     if (L == 0 || nh == 0) return;
     auto s = static_cast<hipStream_t>(stream);
     auto *part = static_cast<float *>(workspace);
+    const bool aligned = (reinterpret_cast<uintptr_t>(out) | reinterpret_cast<uintptr_t>(q) |
+                          reinterpret_cast<uintptr_t>(k) | reinterpret_cast<uintptr_t>(v)) % 16 == 0;
+    if (aligned && selfAttentionMfmaTakes(type, L, S, nkvh, d, dv, scale)) {
+        const auto plan = planSelfAttentionMfma(type, L, S, nh, nkvh, computeUnits());
+        LLAISYS_CHECK(plan.splits == 1 || part, "self_attention: this shape needs selfAttentionWorkspaceBytes() of workspace");
+        selfAttentionMfma(out, q, k, v, type, L, S, nh, nkvh, d, scale, plan, part, s);
+        if (plan.splits > 1) {
+            switch (type) {
+            case ElemType::F32: return merge<float>(out, part, L, nh, dv, plan.splits, s);
+            case ElemType::F16: return merge<__half>(out, part, L, nh, dv, plan.splits, s);
+            case ElemType::BF16: return merge<__hip_bfloat16>(out, part, L, nh, dv, plan.splits, s);
+            }
+        }
+        return;
+    }
     switch (type) {
     case ElemType::F32: return launch<float>(out, q, k, v, L, S, nh, nkvh, d, dv, scale, s, part);
     case ElemType::F16: return launch<__half>(out, q, k, v, L, S, nh, nkvh, d, dv, scale, s, part);
