@@ -64,10 +64,22 @@ void pagedDecode(void *out, bool out_f32, const uint16_t *q, const uint16_t *k_p
 // one launch. For batches whose contexts are of similar length (the waves
 // of a long sequence's workgroup would otherwise finish last). out_packed
 // (bf16 only): the output rows in operand order (packedRowIndex) there
-// instead of in out.
+// instead of in out. keep_invalid: rows of an invalid length stay as they
+// are, as pagedDecode leaves them (else zeros).
 void pagedDecodeUnits(void *out, bool out_f32, const uint16_t *q, const uint16_t *k_pool, const uint16_t *v_pool,
                       const int32_t *block_table, const int32_t *ctx_len, int B, int nh, int nkvh, int max_pages,
-                      int num_blocks, float scale, int *err, void *stream, uint16_t *out_packed = nullptr);
+                      int num_blocks, float scale, int *err, void *stream, uint16_t *out_packed = nullptr,
+                      bool keep_invalid = false);
+// Whether a batch of contexts of up to max_pages pages takes it whatever their
+// spread: one launch instead of two while a unit is short (us, this /
+// stream-K, 12:2 heads): 1 x 300 tokens 5.9 / 8.6, 1 x 700 9.0 / 10.1, 64 x
+// 50-200 5.9 / 9.5, 128 x 64-448 9.2 / 14.2. Past the line a call waits for
+// the one CU of a unit (55 GB/s): 1 x 1500 16.2 / 11.0; with 128 units and
+// more every CU has one, and it lies further out: 64 x 300-800 11.6 / 13.8, 64
+// x 1000-2000 23.6 / 23.6.
+inline bool unitDecodeTakes(int B, int nkvh, int max_pages) {
+    return max_pages <= ((long long)B * nkvh >= 128 ? 64 : 48);
+}
 
 // pagedDecodeUnits with the decode step's QKV epilogue fused in (one token per
 // sequence): from qkv [B, (nh + 2 nkvh) * 128] (projection rows before bias)

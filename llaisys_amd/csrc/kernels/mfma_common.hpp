@@ -58,6 +58,17 @@ __device__ __forceinline__ int waveInclusiveSum(int x) {
     return x;
 }
 
+// Max over the 64 lanes of non-negative x, the same way; the same in all lanes.
+__device__ __forceinline__ int waveMaxInt(int x) {
+    x = max(x, __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, false));
+    x = max(x, __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, false));
+    x = max(x, __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, false));
+    x = max(x, __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, false));
+    x = max(x, __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false));
+    x = max(x, __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false));
+    return __builtin_amdgcn_readlane(x, 63);
+}
+
 // Keeps the 16-bit halves of a word whose key is valid.
 __device__ __forceinline__ uint32_t keepPair(bool lo, bool hi) {
     return (lo ? 0x0000ffffu : 0u) | (hi ? 0xffff0000u : 0u);

@@ -14,7 +14,7 @@
 // (normalised output). Otherwise every wave holding part of it writes a
 // record (unnormalised O, running max m, sum l), and the combine kernel,
 // launched next on the same stream, merges each split unit's records with
-// log-sum-exp weights. A unit spread over at most kUnitSlots waves keeps its
+// log-sum-exp weights. A unit spread over at most `slots` waves keeps its
 // records in slots of its own (slot k = the wave's place among the unit's
 // waves) in a persistent buffer, each with a header holding the record count:
 // the combine then finds them without knowing the lengths, in one memory
@@ -50,7 +50,11 @@ using namespace mfma;
 
 constexpr int kPairsPerWave = 64; // one pair per lane in the wave's block-id window
 constexpr int kMergeBatch = 4;    // records whose loads are in flight together
-constexpr int kUnitSlots = 8;     // per-unit record slots (units spread over more waves use per-wave records)
+// Per-unit record slots (units spread over more waves use per-wave records):
+// kManySlots for batches of up to kManySlotUnits units, whose few sequences
+// are cut into many pieces; kFirstSlots, which the combine requests before it
+// knows how many are used, for larger ones.
+constexpr int kFirstSlots = 8, kManySlots = 32, kManySlotUnits = 512;
 
 struct DecodeArgs {
     const uint16_t *q;
@@ -64,9 +68,10 @@ struct DecodeArgs {
     float *records;
     int *err;
     int *slot_hdr;   // null: every split unit uses the per-wave records
-    float *slot_rec; // kUnitSlots records of G * (kHeadDim + 2) floats per unit
+    float *slot_rec; // `slots` records of G * (kHeadDim + 2) floats per unit
     uint16_t *out_packed; // non-null (bf16 out): rows go there in operand order (packedRowIndex) instead of to out
     int B, T, nh, nkvh, G, max_pages, num_blocks, W;
+    int slots; // record slots per unit
     float scale_log2;
 };
 
@@ -91,11 +96,11 @@ __device__ __forceinline__ void storePackedPieces(uint16_t *dst, int row, int co
 // query rows into Q. Invalid lengths (< 1 or beyond the block table) count as
 // empty and raise kErrTooLong when `report`; so do sequences with more than one
 // query when cu_q is given (they are the prefill kernel's), without an error.
-// Returns the total pair count N. One wave; the caller synchronises before
-// reading S/C/Q from other waves.
-__device__ int scanPairs(const DecodeArgs &a, int *S, int *C, int *Q, bool report) {
+// Returns the total pair count N, and the most pairs of one unit in longest.
+// One wave; the caller synchronises before reading S/C/Q from other waves.
+__device__ int scanPairs(const DecodeArgs &a, int *S, int *C, int *Q, bool report, int &longest) {
     const int lane = threadIdx.x & 63;
-    int carry = 0;
+    int carry = 0, most = 0;
     for (int base = 0; base < a.B; base += 64) {
         const int bb = base + lane;
         int c = 0, row = bb;
@@ -117,7 +122,9 @@ __device__ int scanPairs(const DecodeArgs &a, int *S, int *C, int *Q, bool repor
             }
             if (!mine) c = 0;
         }
-        const int mine_pairs = ((((c + 15) >> 4) + 1) >> 1) * a.nkvh;
+        const int unit_pairs = (((c + 15) >> 4) + 1) >> 1;
+        const int mine_pairs = unit_pairs * a.nkvh;
+        most = max(most, unit_pairs);
         const int incl = waveInclusiveSum(mine_pairs);
         if (bb < a.B) {
             S[bb] = carry + incl - mine_pairs;
@@ -127,12 +134,27 @@ __device__ int scanPairs(const DecodeArgs &a, int *S, int *C, int *Q, bool repor
         carry += __builtin_amdgcn_readlane(incl, 63);
     }
     if (lane == 0) S[a.B] = carry;
+    longest = waveMaxInt(most);
     return carry;
 }
 
-// Slices of P = ceil(N / W) pairs: wave w takes [w P, min((w + 1) P, N)), so
-// only the last waves can be short or empty.
-__device__ __forceinline__ int pairsPerWave(int N, int W) { return (N + W - 1) / W; }
+// Slices of P pairs: wave w takes [w P, min((w + 1) P, N)), so only the last
+// waves can be short or empty. P = ceil(N / W), or more where that would cut
+// the longest unit finer than pays: into over kManySlots pieces (a unit of up
+// to (slots - 1) P pairs touches at most `slots` slices), or into over
+// kFirstSlots, whose merge waits for a second round trip (0.6 us), where up to
+// 3 pairs a wave (0.3 us each) avoid it. A few long sequences over all the
+// waves left a record per page pair, and merging them took longer than the
+// stream; one sequence of 1500 / 4000 / 16000 tokens, 12:2 heads: 15.7 / 27.1
+// / 35.3 us without this rule, 11.0 / 13.0 / 21.6 with it. Larger batches
+// (kFirstSlots) leave the few units that are cut finer to the per-wave records.
+__device__ __forceinline__ int pairsPerWave(const DecodeArgs &a, int N, int longest) {
+    int least = 1;
+    if (a.slots != kFirstSlots)
+        least = max(min(kPairsPerWave, (longest + kManySlots - 2) / (kManySlots - 1)),
+                    min(3, (longest + kFirstSlots - 2) / (kFirstSlots - 1)));
+    return max((N + a.W - 1) / a.W, least);
+}
 __device__ __forceinline__ int waveStart(int w, int N, int P) { return min(w * P, N); }
 // Wave holding pair g (0 <= g < N).
 __device__ __forceinline__ int waveOf(int g, int W, int P) { return min(g / P, W - 1); }
@@ -168,9 +190,10 @@ __global__ void __launch_bounds__(64)
     const int w = blockIdx.x;
     const int G = a.G;
 
-    const int N = scanPairs(a, S, C, Q, w == 0);
+    int longest;
+    const int N = scanPairs(a, S, C, Q, w == 0, longest);
     __syncthreads();
-    const int P = pairsPerWave(N, a.W);
+    const int P = pairsPerWave(a, N, longest);
     const int s = waveStart(w, N, P);
     const int e = waveStart(w + 1, N, P);
     const int cnt = e - s;
@@ -259,18 +282,18 @@ __global__ void __launch_bounds__(64)
         }
         // The unit's records: slot k (this wave's place among the unit's
         // waves) of the unit's own slots with a header holding the record
-        // count, or, past kUnitSlots waves, this wave's per-wave record with
+        // count, or, past `slots` waves, this wave's per-wave record with
         // slot 0's header marking the unit as overflowed (-1).
         const int unit = cur_b * a.nkvh + cur_h;
         const int nrec = first < s ? slot_n[0] : slot_n[1];
         float *rec;
-        if (nrec <= kUnitSlots) {
+        if (nrec <= a.slots) {
             const int k = first < s ? slot_k[0] : slot_k[1];
-            rec = a.slot_rec + size_t(unit * kUnitSlots + k) * G * (kHeadDim + 2);
-            if (lane == 0) a.slot_hdr[unit * kUnitSlots + k] = nrec;
+            rec = a.slot_rec + size_t(unit * a.slots + k) * G * (kHeadDim + 2);
+            if (k == 0 && lane == 0) a.slot_hdr[unit * a.slots] = nrec;
         } else {
             rec = recordAt(a, 2 * w + (first <= s ? 0 : 1));
-            if (a.slot_hdr && first >= s && lane == 0) a.slot_hdr[unit * kUnitSlots] = -1;
+            if (a.slot_hdr && first >= s && lane == 0) a.slot_hdr[unit * a.slots] = -1;
         }
         if (n < G) {
 #pragma unroll
@@ -300,7 +323,7 @@ __global__ void __launch_bounds__(64)
         slot_n[1] = wv(fl + nl - 1) - w0l + 1;
         const bool slots = a.slot_hdr != nullptr;
 #pragma unroll
-        for (int i = 0; i < 2; ++i) slot_n[i] = __builtin_amdgcn_readfirstlane(slots ? slot_n[i] : kUnitSlots + 1);
+        for (int i = 0; i < 2; ++i) slot_n[i] = __builtin_amdgcn_readfirstlane(slots ? slot_n[i] : a.slots + 1);
 #pragma unroll
         for (int i = 0; i < 2; ++i) slot_k[i] = __builtin_amdgcn_readfirstlane(slot_k[i]);
     }
@@ -335,8 +358,8 @@ __global__ void __launch_bounds__(64)
 
 // Merge the records of every unit that spans more than one wave.
 // 256 threads = 4 waves per unit. With record slots, wave v loads slots 2v
-// and 2v+1 with their headers (and every wave slot 0's header) in one go and
-// merges the valid ones. Without them (or for an overflowed unit) wave 0
+// and 2v+1 with slot 0's header (the unit's record count) in one go, and the
+// slots past kFirstSlots that the count asks for after it. Without them (or for an overflowed unit) wave 0
 // scans the lengths into LDS, lane k works out which per-wave record k of the
 // unit lives in (the integer divisions run lane-parallel), and wave v takes
 // records v, v+4, ... in batches with all loads of a batch in flight. Merging
@@ -366,32 +389,34 @@ __global__ void __launch_bounds__(64 * kCombineWaves) decodeCombineKernel(Decode
 #pragma unroll
     for (int i = 0; i < 8; ++i) o[i] = f32x4{0.f, 0.f, 0.f, 0.f};
     int row;
-    int clear_mask = 0; // this wave's slots whose headers go back to zero (after the barrier below)
+    bool clear = false; // the unit's header goes back to zero (after the barrier below)
     bool per_wave = a.slot_hdr == nullptr;
     if (!per_wave) {
-        // The unit's slots: wave v takes slots 2v and 2v+1. Headers, records
-        // and the output row are all requested before any of them is used, so
-        // the merge waits for one memory round trip.
-        int *hdr = a.slot_hdr + u * kUnitSlots;
+        // The unit's slots: wave v takes slots 2v and 2v+1 of every
+        // kFirstSlots. The count, the first records and the output row are
+        // all requested before any of them is used, so the merge of up to
+        // kFirstSlots records waits for one memory round trip.
+        const int *hdr = a.slot_hdr + u * a.slots;
         const int h0 = hdr[0];
-        int hk[2];
         float2 ml[2];
         f32x4 orr[2][8];
-#pragma unroll
-        for (int t = 0; t < 2; ++t) {
-            const int k = 2 * wave + t;
-            hk[t] = hdr[k];
-            const float *rec = a.slot_rec + size_t(u * kUnitSlots + k) * G * (kHeadDim + 2);
-            ml[t] = *reinterpret_cast<const float2 *>(rec + recordML(G, col));
-#pragma unroll
-            for (int i = 0; i < 8; ++i) orr[t][i] = *reinterpret_cast<const f32x4 *>(rec + recordO(G, i, col, grp));
-        }
-        row = a.cu_q ? a.cu_q[b] : b;
-        if (h0 == 0) return; // unit whole in one wave (or not a decode row): nothing to merge
-        if (h0 > 0) {
+        auto request = [&](int k0) {
 #pragma unroll
             for (int t = 0; t < 2; ++t) {
-                if (hk[t] <= 0 || ml[t].x == -INFINITY) continue;
+                const float *rec = a.slot_rec + size_t(u * a.slots + k0 + 2 * wave + t) * G * (kHeadDim + 2);
+                ml[t] = *reinterpret_cast<const float2 *>(rec + recordML(G, col));
+#pragma unroll
+                for (int i = 0; i < 8; ++i) orr[t][i] = *reinterpret_cast<const f32x4 *>(rec + recordO(G, i, col, grp));
+            }
+        };
+        request(0);
+        row = a.cu_q ? a.cu_q[b] : b;
+        if (h0 == 0) return; // unit whole in one wave (or not a decode row): nothing to merge
+        for (int k0 = 0; k0 < h0; k0 += kFirstSlots) {
+            if (k0) request(k0);
+#pragma unroll
+            for (int t = 0; t < 2; ++t) {
+                if (k0 + 2 * wave + t >= h0 || ml[t].x == -INFINITY) continue;
                 const float Mn = fmaxf(M, ml[t].x);
                 const float sa = exp2Fast(M - Mn);
                 const float sb = exp2Fast(ml[t].x - Mn);
@@ -400,21 +425,24 @@ __global__ void __launch_bounds__(64 * kCombineWaves) decodeCombineKernel(Decode
                 for (int i = 0; i < 8; ++i) o[i] = o[i] * sa + orr[t][i] * sb;
                 M = Mn;
             }
-            clear_mask = (hk[0] != 0 ? 1 : 0) | (hk[1] != 0 ? 2 : 0);
-        } else {
-            per_wave = true; // overflowed: per-wave records
-            clear_mask = wave == 0 ? 1 : 0;
         }
+        per_wave = h0 < 0; // overflowed: per-wave records
+        clear = true;
     }
     if (per_wave) {
-        if (wave == 0) scanPairs(a, S, C, Q, false);
+        __shared__ int s_longest;
+        if (wave == 0) {
+            int longest;
+            scanPairs(a, S, C, Q, false, longest);
+            if (lane == 0) s_longest = longest;
+        }
         __syncthreads();
         const int N = S[a.B];
         const int np = (C[b] + 15) >> 4;
         const int npr = (np + 1) >> 1;
         if (npr == 0) return;
         const int first = S[b] + h * npr;
-        const int P = pairsPerWave(N, a.W);
+        const int P = pairsPerWave(a, N, s_longest);
         const int w0 = waveOf(first, a.W, P);
         const int w1 = waveOf(first + npr - 1, a.W, P);
         if (w0 == w1) return;
@@ -467,13 +495,9 @@ __global__ void __launch_bounds__(64 * kCombineWaves) decodeCombineKernel(Decode
         part_ml[wave - 1][1][lane] = L;
     }
     __syncthreads();
-    // Every wave has read the unit's headers by now: leave them at zero for
-    // the next call.
-    if (clear_mask && lane == 0) {
-        int *hdr = a.slot_hdr + u * kUnitSlots + 2 * wave;
-        if (clear_mask & 1) hdr[0] = 0;
-        if (clear_mask & 2) hdr[1] = 0;
-    }
+    // Every wave has read the unit's header by now: leave it at zero for the
+    // next call.
+    if (clear && threadIdx.x == 0) a.slot_hdr[u * a.slots] = 0;
     if (wave > 0 || n >= G) return;
 #pragma unroll
     for (int v = 0; v < kCombineWaves - 1; ++v) {
@@ -566,6 +590,7 @@ struct RopeArgs {
     int hs;
     float eps, theta;
     uint16_t *o_packed; // non-null: the output rows go there in operand order (with or without ROPE)
+    bool keep_invalid;  // an invalid length leaves its output rows alone (else zeros)
 };
 
 template <bool OUT_F32, int NSTAGE, bool ROPE>
@@ -805,7 +830,7 @@ __global__ void __launch_bounds__(64 * kUnitWaves)
         part_ml[wave - 1][1][lane] = lt;
     }
     __syncthreads();
-    if (wave > 0 || n >= G) return;
+    if (wave > 0 || n >= G || (c == 0 && r.keep_invalid)) return;
     float M = acc.m, L = lt;
 #pragma unroll
     for (int v = 0; v < kUnitWaves - 1; ++v) {
@@ -914,12 +939,22 @@ void pagedDecodeNoAlloc(void *out, bool out_f32, const uint16_t *q, const uint16
                       "paged_attention_no_alloc: " << Bc << " sequences x " << nkvh << " kv heads x " << max_pages
                           << " pages need " << plan.record_bytes << " bytes of split records, more than the "
                           << kNoAllocScratchBytes << "-byte scratch; use llaisysPagedAttention");
+        if (unitDecodeTakes(Bc, nkvh, max_pages)) {
+            pagedDecodeUnits(static_cast<std::byte *>(out) + size_t(b0) * nh * kHeadDim * esz, out_f32,
+                             q + size_t(b0) * nh * kHeadDim, k_pool, v_pool, block_table + size_t(b0) * max_pages,
+                             ctx_len + b0, Bc, nh, nkvh, max_pages, num_blocks, scale, err, stream, nullptr, true);
+            continue;
+        }
         pagedDecode(static_cast<std::byte *>(out) + size_t(b0) * nh * kHeadDim * esz, out_f32,
                     q + size_t(b0) * nh * kHeadDim, k_pool, v_pool, block_table + size_t(b0) * max_pages,
                     ctx_len + b0, nullptr, Bc, Bc, nh, nkvh, max_pages, num_blocks, scale, plan,
                     static_cast<float *>(ptr), err, nullptr, nullptr, stream);
     }
 }
+
+namespace {
+int slotsFor(int B, int nkvh) { return (long long)B * nkvh <= kManySlotUnits ? kManySlots : kFirstSlots; }
+} // namespace
 
 DecodePlan planDecode(int B, int nkvh, int group, int max_pages) {
     DecodePlan p{};
@@ -934,7 +969,7 @@ DecodePlan planDecode(int B, int nkvh, int group, int max_pages) {
     p.lds_bytes = size_t(3 * B + 1) * sizeof(int);
     p.stages = envInt("LLAISYS_DECODE_STAGES", 2) >= 3 ? 3 : 2;
     // Per-unit record slots, unless disabled or implausibly large.
-    const size_t slots = size_t(B) * nkvh * kUnitSlots;
+    const size_t slots = size_t(B) * nkvh * slotsFor(B, nkvh);
     const size_t rec_bytes = slots * group * (kHeadDim + 2) * sizeof(float);
     const bool use = envInt("LLAISYS_DECODE_SLOTS", 1) != 0 && rec_bytes <= (size_t(1) << 30);
     p.slot_headers = use ? slots : 0;
@@ -964,6 +999,7 @@ void pagedDecode(void *out, bool out_f32, const uint16_t *q, const uint16_t *k_p
     const bool slots = plan.slot_headers && slot_headers && slot_records;
     a.slot_hdr = slots ? slot_headers : nullptr;
     a.slot_rec = slots ? static_cast<float *>(slot_records) : nullptr;
+    a.slots = slotsFor(B, nkvh);
     a.B = B;
     a.T = T;
     a.nh = nh;
@@ -1041,11 +1077,12 @@ void launchDecodeUnits(void *out, bool out_f32, const uint16_t *q, const uint16_
 
 void pagedDecodeUnits(void *out, bool out_f32, const uint16_t *q, const uint16_t *k_pool, const uint16_t *v_pool,
                       const int32_t *block_table, const int32_t *ctx_len, int B, int nh, int nkvh, int max_pages,
-                      int num_blocks, float scale, int *err, void *stream, uint16_t *out_packed) {
+                      int num_blocks, float scale, int *err, void *stream, uint16_t *out_packed, bool keep_invalid) {
     LLAISYS_CHECK(!out_packed || (!out_f32 && (nh * kHeadDim) % 32 == 0),
                   "pagedDecodeUnits: a packed output is bf16 with nh * 128 % 32 == 0");
     RopeArgs r{};
     r.o_packed = out_packed;
+    r.keep_invalid = keep_invalid;
     launchDecodeUnits(out, out_f32, q, k_pool, v_pool, block_table, ctx_len, B, nh, nkvh, max_pages, num_blocks,
                       scale, err, r, false, stream);
 }
@@ -1064,7 +1101,7 @@ void pagedDecodeUnitsRope(void *out, bool out_f32, uint16_t *k_pool, uint16_t *v
     LLAISYS_CHECK(!x || (hs > 0 && hs % 8 == 0), "pagedDecodeUnitsRope: hidden size must be a positive multiple of 8");
     LLAISYS_CHECK(!out_packed || (!out_f32 && (nh * kHeadDim) % 32 == 0),
                   "pagedDecodeUnitsRope: a packed output is bf16 with nh * 128 % 32 == 0");
-    const RopeArgs r{qkv, bias, x, k_pool, v_pool, hs, eps, theta, out_packed};
+    const RopeArgs r{qkv, bias, x, k_pool, v_pool, hs, eps, theta, out_packed, false};
     launchDecodeUnits(out, out_f32, nullptr, k_pool, v_pool, block_table, ctx_len, B, nh, nkvh, max_pages,
                       num_blocks, scale, err, r, true, stream);
 }

@@ -192,13 +192,15 @@ Qwen2Model::DecodeGraph Qwen2Model::capture(const std::function<void()> &work, s
 // Decode steps (B > 0) of at least kUnitDecodeMinUnits units whose lengths
 // stay within 2x: every unit's workgroup then finishes at about the same
 // time, and the one-launch kernel saves the stream-K kernel's length scan,
-// split records and combine launch. Other batches (mixed lengths, few
-// sequences, prefill) keep the stream-K kernel.
+// split records and combine launch. So do batches of short contexts, whatever
+// their number and spread. Other batches (mixed lengths, few sequences,
+// prefill) keep the stream-K kernel.
 static constexpr size_t kUnitDecodeMinUnits = 128;
 
 void Qwen2Model::chooseDecodeAttention(size_t B, int32_t min_ctx, int32_t max_ctx) {
-    unit_decode_ = unit_decode_allowed_ && B > 0 && B * cfg_.nkvh >= kUnitDecodeMinUnits && min_ctx >= 1 &&
-                   max_ctx <= 2 * min_ctx;
+    const bool similar = B * cfg_.nkvh >= kUnitDecodeMinUnits && max_ctx <= 2 * min_ctx;
+    unit_decode_ = unit_decode_allowed_ && B > 0 && min_ctx >= 1 &&
+                   (similar || K::unitDecodeTakes(int(B), int(cfg_.nkvh), (max_ctx + K::kPageTokens - 1) / K::kPageTokens));
 }
 
 void Qwen2Model::decodeGraph(size_t B, size_t width) {

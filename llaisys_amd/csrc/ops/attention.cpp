@@ -319,6 +319,11 @@ void pagedAttention(const tensor_t &out, const tensor_t &q, const tensor_t &k_po
     const auto *tab = reinterpret_cast<const int32_t *>(block_table->data());
     const auto *ctx = reinterpret_cast<const int32_t *>(ctx_len->data());
     const int nb = int(k_pool->shape()[0]);
+    if (!cu_q && K::unitDecodeTakes(int(B), int(nkvh), max_pages)) {
+        K::pagedDecodeUnits(out->data(), f32, qp, kp, vp, tab, ctx, int(B), int(nh), int(nkvh), max_pages, nb, scale,
+                            rt.errorWord(), rt.stream(), nullptr, true);
+        return;
+    }
     if (!cu_q) {
         // Decode: sequences are independent, so large batches run in chunks
         // whose length prefix fits the kernel's LDS.
