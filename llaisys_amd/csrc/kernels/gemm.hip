@@ -46,7 +46,6 @@
 #include <algorithm>
 #include <cstdlib>
 #include <mutex>
-#include <type_traits>
 #include <vector>
 
 namespace llaisys::kernels {
@@ -599,6 +598,89 @@ __global__ void __launch_bounds__(256) gemmReduceKernel(void *y, const float *pa
     }
 }
 
+// Few rows of X (M <= 16 MT): W is streamed once by many small workgroups and
+// nothing is staged. A workgroup of NW waves owns R rows of W; its waves take
+// the rows' 128 B segments in turn, straight from memory into MFMA operands.
+// Where M <= R < 16 the MFMA's 16 x 16 would be mostly empty, so its rows and
+// columns are KR = 16 / R groups that take different segments: row group a
+// and column group a meet in the quadrants (a, a), the others are unused, and
+// a workgroup owns fewer rows, so that more of them share a narrow W. The
+// NW KR partial sums of an output meet in LDS in a fixed order.
+template <ElemType T, int R, int NW, int MT>
+__global__ void __launch_bounds__(64 * NW) gemmFewRowsKernel(GemmParams p) {
+    static_assert(MT == 1 || R == 16, "column groups are of one tile");
+    constexpr int KR = 16 / R, U = MT == 1 ? 4 : 2; // segments in flight per set
+    __shared__ float part[NW * KR][MT * R][R];
+    const int lane = threadIdx.x & 63, n = lane & 15, grp = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int n0 = int(blockIdx.x) * R;
+    const __amdgpu_buffer_rsrc_t xr =
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p.x), (short)0, int(p.x_bytes), kRsrcWord3);
+    const __amdgpu_buffer_rsrc_t wr =
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p.w), (short)0, int(p.w_bytes), kRsrcWord3);
+    const uint32_t row_bytes = uint32_t(p.K) * Elem<T>::size;
+    const int segs = int((row_bytes + 127) / 128), steps = (segs + NW * KR - 1) / (NW * KR);
+    // Rows of W past N are past the buffer (zeros); columns past M repeat row 0.
+    const uint32_t wbase = uint32_t(n0 + n % R) * row_bytes;
+    uint32_t xbase[MT];
+#pragma unroll
+    for (int t = 0; t < MT; ++t) xbase[t] = t * 16 + n % R < p.M ? uint32_t(t * 16 + n % R) * row_bytes : 0;
+    struct Set {
+        u32x4 w[U][2], x[U][MT][2];
+    };
+    auto load = [&](Set &f, int step) {
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                const uint32_t k = uint32_t(((step + u) * NW + wave) * KR + n / R) * 128 + 32 * grp + 16 * j;
+                const bool in = k < row_bytes;
+                f.w[u][j] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(wr, int(in ? wbase + k : kMasked), 0, 0));
+#pragma unroll
+                for (int t = 0; t < MT; ++t)
+                    f.x[u][t][j] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(xr, int(in ? xbase[t] + k : kMasked), 0, 0));
+            }
+    };
+    f32x4 acc[MT];
+#pragma unroll
+    for (int t = 0; t < MT; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+    auto use = [&](const Set &f) {
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+#pragma unroll
+                for (int t = 0; t < MT; ++t) acc[t] = mfmaPiece<T>(f.w[u][j], f.x[u][t][j], acc[t]);
+    };
+    Set a, b;
+    load(a, 0);
+    for (int s = 0; s < steps; s += 2 * U) {
+        if (s + U < steps) load(b, s + U);
+        use(a);
+        if (s + U >= steps) break;
+        if (s + 2 * U < steps) load(a, s + 2 * U);
+        use(b);
+    }
+    // Lane: rows 4 grp + i of the tile, column n; in quadrant (a, a) both belong to group a.
+    if ((4 * grp) / R == n / R) {
+#pragma unroll
+        for (int t = 0; t < MT; ++t)
+            *reinterpret_cast<f32x4 *>(&part[wave * KR + n / R][t * R + n % R][(4 * grp) % R]) = acc[t];
+    }
+    __syncthreads();
+    for (int i = threadIdx.x; i < MT * R * R; i += 64 * NW) {
+        const int m = i / R, r = i % R;
+        if (m >= p.M || n0 + r >= p.N) continue;
+        float v = part[0][m][r];
+#pragma unroll
+        for (int s = 1; s < NW * KR; ++s) v += part[s][m][r];
+        const size_t at = size_t(m) * p.ldy + n0 + r;
+        if (p.accumulate) v = loadElem<T>(p.y, at) + v;
+        if (p.bias) v += loadElem<T>(p.bias, n0 + r);
+        storeElem<T>(p.y, at, v);
+    }
+}
+
 int cusOf() {
     static std::mutex mu;
     static std::vector<int> cache;
@@ -775,6 +857,40 @@ bool w8() {
     return v;
 }
 
+// Where the few-rows kernel runs. us, this / the tiled GEMM (with its K split
+// and reduce launch), N x K, MI355X; 4.5 is what the calls themselves take:
+//   16-bit        1536 x 1536  8960 x 1536  17920 x 1536  1536 x 8960  151936 x 1536
+//   M = 1          4.5 /  7.4   7.1 /  9.2   11.4 / 13.7   7.8 / 11.3   78.6 / 100.8
+//   M = 5          4.5 /  7.1   9.0 /  9.2   13.9 / 13.8   9.6 / 11.4    106 / 101
+//   M = 16         5.1 /  7.2  10.9 /  9.3   16.0 / 13.9  18.3 / 12.1    118 / 104
+//   M = 30         6.3 /  7.2  14.5 /  9.5   22.3 / 14.4  25.3 / 12.1
+//   f32, M = 1     4.8 /  9.9  13.0 / 32.5                14.6 / 28.2
+//   M = 5          5.9 / 10.4  16.0 / 32.9                17.4 / 28.4
+//   M = 16         8.5 / 10.8  19.0 / 33.4                34.3 / 28.7
+// Every workgroup reads the rows of X for its few rows of W, so with M the
+// lead goes to the tiles, first where W is large.
+bool takesFewRows(ElemType t, const GemmParams &p) {
+    const long nk = long(p.N) * p.K;
+    if ((reinterpret_cast<uintptr_t>(p.x) | reinterpret_cast<uintptr_t>(p.w)) % 16 || p.swiglu) return false;
+    if (p.M <= 4) return true;
+    if (t == ElemType::F32) return p.M <= 8 || (p.M <= 16 && p.K <= 4096);
+    return (p.M <= 8 && p.N <= 4096) || (p.M <= 32 && nk <= (1L << 22));
+}
+
+template <ElemType T, int R, int NW, int MT> void launchFewRowsAs(const GemmParams &p, hipStream_t s) {
+    hipLaunchKernelGGL((gemmFewRowsKernel<T, R, NW, MT>), dim3(unsigned((p.N + R - 1) / R)), dim3(64 * NW), 0, s, p);
+    HIP_CHECK(hipGetLastError());
+}
+
+// 2 waves a workgroup for the 16-bit rows of M <= 4, else 4 (8 were slower on
+// wide W: half of them had no segment at K = 1536).
+template <ElemType T> void launchFewRows(const GemmParams &p, hipStream_t s) {
+    if (p.M <= 4) launchFewRowsAs<T, 4, Elem<T>::size == 4 ? 4 : 2, 1>(p, s);
+    else if (p.M <= 8) launchFewRowsAs<T, 8, 4, 1>(p, s);
+    else if (p.M <= 16) launchFewRowsAs<T, 16, 4, 1>(p, s);
+    else launchFewRowsAs<T, 16, 4, 2>(p, s);
+}
+
 template <ElemType T> void launchGemm(GemmParams p, const Plan &plan, hipStream_t s) {
     p.mtiles = plan.mtiles;
     p.ntiles = plan.ntiles;
@@ -877,6 +993,28 @@ void linear(void *y, const void *x, const void *w, const void *bias, ElemType t,
     const int rows_per_launch = rowsPerLaunch(t, M, K);
     for (int r0 = 0; r0 < M; r0 += rows_per_launch) {
         const int m = std::min(rows_per_launch, M - r0);
+        if (m <= 32) {
+            GemmParams p{};
+            p.y = static_cast<char *>(y) + size_t(r0) * N * es;
+            p.x = static_cast<const char *>(x) + size_t(r0) * row_bytes;
+            p.w = w;
+            p.bias = bias;
+            p.M = m;
+            p.N = N;
+            p.K = K;
+            p.ldy = N;
+            p.accumulate = accumulate ? 1 : 0;
+            p.x_bytes = uint32_t(size_t(m) * row_bytes);
+            p.w_bytes = uint32_t(size_t(N) * row_bytes);
+            if (takesFewRows(t, p)) {
+                switch (t) {
+                case ElemType::BF16: launchFewRows<ElemType::BF16>(p, s); break;
+                case ElemType::F16: launchFewRows<ElemType::F16>(p, s); break;
+                case ElemType::F32: launchFewRows<ElemType::F32>(p, s); break;
+                }
+                continue;
+            }
+        }
         const Plan plan = planGemm(t, m, N, K);
         LLAISYS_CHECK(plan.splits == 1 || workspace, "linear: this shape needs linearWorkspaceBytes() of workspace");
         // Columns [c0, c1) of this launch's rows on `pl` (y keeps its row stride N).
