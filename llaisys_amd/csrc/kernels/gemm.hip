@@ -184,14 +184,15 @@ __device__ __forceinline__ int slotOf(int r, int c) { return c ^ rowKey(r); }
 // against 503 and 497 us; more loads in flight per CU than it can stream).
 template <bool PIPE, int RB = 64, int WS = 2> constexpr int ringStages() { return RB == 128 ? WS : 4; }
 
-// Stages of the wide ring: two for the 8-wave tiles (256 x 256 and 256 x 192
-// fit no more; 128 x 256 and 256 x 128 ran 1-6 % slower with three), four
-// for the 4-wave ones, whose short k loops wait on their loads more: 1024 x
+// Stages of the wide ring: what fits, up to four: two for 256 x 256 and 256 x
+// 192, three for 128 x 256 and 256 x 128 (200 x 17920 x 1536 29.2 -> 25.2 us
+// against two, now that the loads go out between the reads), four for the
+// 4-wave tiles, whose short k loops wait on their loads more: 1024 x
 // 2048 x 1536 16.9 -> 14.1 us, 1024 x 1536 x 8960 47.6 -> 37.4 us, 2048 x 1536
 // x 1536 17.1 -> 14.8 us (LLAISYS_GEMM_WIDE_DEEP=0: two everywhere).
 template <int BM, int BN, int NW> constexpr int wideStages() {
     constexpr int n = 163840 / (((BM / 8) + (BN / 8 + NW - 1) / NW * NW) * 1024);
-    return NW > 4 ? 2 : n > 4 ? 4 : n < 2 ? 2 : n;
+    return n > 4 ? 4 : n < 2 ? 2 : n;
 }
 
 // Wide k tiles (RB = 128: 64 16-bit k per row and stage). A 64 B row piece
@@ -250,19 +251,24 @@ __global__ void __launch_bounds__(64 * WGM * WGN) gemmKernel(GemmParams p) {
     const int nk_all = (p.K + KT - 1) / KT;
     const int kt0 = split * nk_all / p.splits;
     const int nk = (split + 1) * nk_all / p.splits - kt0;
-    auto issue = [&](int kt) {
+    // Load l of the wave's kLoadsPerStage of k tile kt: X blocks, then W blocks.
+    auto issueOne = [&](int kt, int l) {
         u32x4 *st = lds + (kt % NS) * STAGE;
         const uint32_t kb = uint32_t(kt0 + kt) * RB;
         const bool in_k = kt < nk && kb + 16 * lc < row_bytes;
-#pragma unroll
-        for (int b = 0; b < XW; ++b)
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(xr, (lds_void *)(st + (wave + NW * b) * 64), 16,
-                                                     int(in_k ? xbase + kb + b * bstride : kMasked), 0, 0, 0);
-#pragma unroll
-        for (int b = 0; b < WW; ++b)
+        if (l < XW) {
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(xr, (lds_void *)(st + (wave + NW * l) * 64), 16,
+                                                     int(in_k ? xbase + kb + l * bstride : kMasked), 0, 0, 0);
+        } else {
+            const int b = l - XW;
             __builtin_amdgcn_raw_ptr_buffer_load_lds(
                 wr, (lds_void *)(st + (XB + wave + NW * b) * 64), 16,
                 int(in_k && (WB % NW == 0 || wave + NW * b < WB) ? wbase + kb + b * bstride : kMasked), 0, 0, 0);
+        }
+    };
+    auto issue = [&](int kt) {
+#pragma unroll
+        for (int l = 0; l < kLoadsPerStage; ++l) issueOne(kt, l);
     };
 
     f32x4 acc[TN][TM];
@@ -326,6 +332,34 @@ __global__ void __launch_bounds__(64 * WGM * WGN) gemmKernel(GemmParams p) {
                 __builtin_amdgcn_sched_group_barrier(0x008, kPer, 0); // then MFMAs
             }
         };
+        // The first half of stage kt with the loads of stage ki between its
+        // reads (the compiler keeps LDS reads and loads to LDS in order). Sent
+        // all at once after the barrier, the loads of the CU's waves queued
+        // ahead of the reads that the next MFMAs wait for: 8192 x 17920 x 1536
+        // 395 -> 380 us (1185 TFLOP/s), x 6144 1414 -> 1350 (1335), 4000 x 5000
+        // x 2048 87 -> 80.
+        constexpr int kAt = (kLoadsPerStage + kReads - 1) / kReads; // loads after a read
+        auto readHalfIssue = [&](int kt, int ki, u32x4 (&a)[TN], u32x4 (&b)[TM]) {
+            const u32x4 *st = lds + (kt % NS) * STAGE;
+            const int slot = (lane >> 4) ^ (fr & 7);
+#pragma unroll
+            for (int g = 0; g < kReads; ++g) {
+                if (g < TN)
+                    a[g] = st[(BM + 16 * (wn * TN + g) + fr) * PPR + slot];
+                else
+                    b[g - TN] = st[(16 * (wm * TM + g - TN) + fr) * PPR + slot];
+#pragma unroll
+                for (int l = g * kAt; l < (g + 1) * kAt && l < kLoadsPerStage; ++l) issueOne(ki, l);
+            }
+        };
+        auto interleaveLoads = [&]() {
+#pragma unroll
+            for (int g = 0; g < kReads; ++g) {
+                __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);    // one LDS read
+                if (g * kAt < kLoadsPerStage) __builtin_amdgcn_sched_group_barrier(0x010, kAt, 0); // loads of the ring
+                __builtin_amdgcn_sched_group_barrier(0x008, kPer, 0); // then MFMAs
+            }
+        };
         // Stage 0 has landed once only stages 1 .. NS - 1 are in flight.
         asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((NS - 1) * kLoadsPerStage) : "memory");
         u32x4 a0[TN], b0[TM], a1[TN], b1[TM];
@@ -338,10 +372,9 @@ __global__ void __launch_bounds__(64 * WGM * WGN) gemmKernel(GemmParams p) {
             // wave's) and every wave has read all of stage kt, whose slot
             // stage kt + NS takes.
             asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((NS - 2) * kLoadsPerStage) : "memory");
-            issue(kt + NS);
-            readHalf(kt + 1, 0, a0, b0); // past the end: the zero-filled stage
+            readHalfIssue(kt + 1, kt + NS, a0, b0); // past the end: the zero-filled stage
             mfmaTile(a1, b1);
-            interleave();
+            interleaveLoads();
         }
     } else if constexpr (PIPE) {
         // Stage 0 has landed once at most NS - 2 stages are in flight.
