@@ -779,37 +779,53 @@ template <ElemType T, int BM, int BN, int WGM = 2, int WGN = 2> void launchTile(
 }
 
 // The (tile, K split) with the least estimated time. A launch runs
-// ceil(workgroups / CUs) rounds; a round costs a fixed kFixedUs (first loads,
-// epilogue) plus the tile's k loop, bm x bn x (K / split) at the tile's
-// relative MFMA rate eff (bigger wave tiles read less LDS per MFMA); a split
-// adds the reduce kernel, priced by its bytes (fp32 partials written and read
-// back, the output written). Fitted to timings of the kernel on MI355X
-// (bf16, M = 2048 / 8192 by the Qwen2 projection widths): e.g. 2048 x 2048 x
-// 1536 runs 21.0 us on 128 x 128 tiles against 29 us on 128 x 256 tiles split
-// in two, and 2048 x 1536 x 8960 85.8 us split in two against 93.5 us not.
+// ceil(workgroups / CUs) rounds; a round takes the tile's fixed time (first
+// loads, epilogue) and its k loop, `step` us per 64 k; two 64 x 64 workgroups
+// share a CU, whose second one adds kShare of a k loop. A split adds the
+// reduce kernel, priced by its bytes (fp32 partials written and read back, the
+// output written). The numbers are fits to 2800 timings on MI355X, 16-bit and
+// f32, M 20-3000 by eight N x K, each tile with 1 to 8 splits (10 % off a
+// timing at the median); the plans they choose take 1.5 % longer than the
+// best ones timed. Splits of any number matter where the tiles of one round
+// leave CUs idle (us, with powers of two and one rate for all tiles before):
+// 777 x 1536 x 8960 40.2 -> 34.7 (128 x 128 in 3), 3000 x 1536 x 8960 102 -> 92
+// (256 x 256 in 3), f32 1024 x 1536 x 1536 99 -> 53, 400 x 8960 x 1536 187 -> 103.
 struct Plan {
     int tile = 0; // index into kTiles
     int mtiles = 0, ntiles = 0, splits = 1;
     double est = 0; // the model's time, us
 };
-// narrow: waves 48 columns wide. 256 x 192 (8 waves of 128 x 48) and
-// 128 x 96 (4 waves of 64 x 48) fill the 256 CUs where the tiles twice their
-// size leave a quarter idle (8192 x 1536 x 1536: 256 tiles against 192, 44.6
-// -> 40.2 us; 2048 x 1536 x 8960 split in 4: 76 -> 69.5 us). They run only
-// where one round holds all their workgroups: over several (2048 x 17920 x
-// 1536: 3 rounds, 128-131 us) 256 x 256 tiles with the column split below run
-// faster (123-125 us) than the model prices them. Their wave columns are not
-// whole SwiGLU block pairs, so the fused gate-up skips them.
-struct TileShape { int bm, bn; double eff; bool narrow; };
-constexpr TileShape kTiles[] = {{128, 256, 1.0, false}, {256, 128, 1.0, false}, {128, 128, 0.8, false},
-                                {64, 64, 0.45, false},  {256, 256, 1.2, false}, {256, 192, 1.1, true},
-                                {128, 96, 0.7, true}};
-constexpr int kTile192 = 5, kTile96 = 6;
-constexpr int kMinSplitTiles = 8;            // k tiles per split at least
-constexpr double kFixedUs = 6.0;             // per round of workgroups
-constexpr double kMacsPerUs = 2.1e6;         // bm * bn * k per us at eff 1 (bf16)
-constexpr double kReduceBytesPerUs = 5.0e6;  // HBM rate of the reduce kernel
-constexpr double kReduceLaunchUs = 2.0;
+// narrow: waves 48 columns wide, not whole SwiGLU block pairs, so the fused
+// gate-up skips them. 256 x 192 (8 waves of 128 x 48) and 128 x 96 (4 waves of
+// 64 x 48) fill the 256 CUs where the tiles twice their size leave a quarter
+// idle (8192 x 1536 x 1536: 256 tiles against 192, 44.6 -> 40.2 us).
+struct TileShape {
+    int bm, bn;
+    bool narrow;
+    double fixed16, step16, step32; // us; f32 runs the first four shapes, kFixed32 fixed
+};
+constexpr TileShape kTiles[] = {{128, 256, false, 5.2, 0.618, 7.5}, {256, 128, false, 4.6, 0.629, 7.5},
+                                {128, 128, false, 4.4, 0.394, 3.95}, {64, 64, false, 3.7, 0.201, 1.08},
+                                {256, 256, false, 6.0, 1.135, 0},    {256, 192, true, 4.7, 0.879, 0},
+                                {128, 96, true, 3.9, 0.350, 0}};
+constexpr int kTile64 = 3, kTile192 = 5, kTile96 = 6;
+constexpr double kFixed32 = 2.0;
+constexpr double kShare = 0.8;             // 16-bit; f32's MFMAs leave nothing to share
+constexpr int kMinSplitTiles = 8;            // k tiles (of 64 B) per split at least
+constexpr int kMaxSplits = 8;
+constexpr double kReduceBytesPerUs = 5.0e6;
+constexpr double kReduceLaunchUs = 2.5;
+
+double roundsUs(ElemType t, int tile, long workgroups, long cus, double k) {
+    const TileShape &c = kTiles[tile];
+    const bool f32 = t == ElemType::F32;
+    const double fixed = f32 ? kFixed32 : c.fixed16, loop = k / 64.0 * (f32 ? c.step32 : c.step16);
+    if (tile != kTile64 || f32) return double((workgroups + cus - 1) / cus) * (fixed + loop);
+    const long rest = workgroups % (2 * cus);
+    double us = double(workgroups / (2 * cus)) * (fixed + (1.0 + kShare) * loop);
+    if (rest) us += fixed + (rest > cus ? 1.0 + kShare : 1.0) * loop;
+    return us;
+}
 
 Plan planGemm(ElemType t, int M, int N, int K, bool no_split = false, bool swiglu = false) {
     const long cus = cusOf();
@@ -826,11 +842,9 @@ Plan planGemm(ElemType t, int M, int N, int K, bool no_split = false, bool swigl
         if ((i == 4 && !big) || (kTiles[i].narrow && (!narrow || swiglu))) continue;
         const TileShape &c = kTiles[i];
         const long mt = (M + c.bm - 1) / c.bm, nt = (N + c.bn - 1) / c.bn;
-        for (int sp = 1; sp <= 8; sp *= 2) {
+        for (int sp = 1; sp <= kMaxSplits; ++sp) {
             if (sp > 1 && (no_split || nk / sp < kMinSplitTiles)) break;
-            const long rounds = (mt * nt * sp + cus - 1) / cus;
-            if (c.narrow && rounds > 1) continue;
-            double tm = double(rounds) * (kFixedUs + double(c.bm) * c.bn * (double(K) / sp) / (c.eff * kMacsPerUs));
+            double tm = roundsUs(t, i, mt * nt * sp, cus, double(K) / sp);
             if (sp > 1)
                 tm += kReduceLaunchUs + (2.0 * sp * 4.0 + es) * double(M) * N / kReduceBytesPerUs;
             if (tm < best_t) {
