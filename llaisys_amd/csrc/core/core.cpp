@@ -116,10 +116,11 @@ int *Runtime::errorWord() {
 }
 
 int *Runtime::queueCounters() {
+    constexpr size_t kQueueWords = kernels::kPrefillQueueWords;
     LLAISYS_CHECK(type_ == LLAISYS_DEVICE_AMD, "device workspace exists on AMD runtimes only");
     if (!queue_counters_) {
-        queue_counters_ = static_cast<int *>(api_->malloc_device(2 * sizeof(int)));
-        if (hipMemset(queue_counters_, 0, 2 * sizeof(int)) != hipSuccess) LLAISYS_RAISE("hipMemset failed");
+        queue_counters_ = static_cast<int *>(api_->malloc_device(kQueueWords * sizeof(int)));
+        if (hipMemset(queue_counters_, 0, kQueueWords * sizeof(int)) != hipSuccess) LLAISYS_RAISE("hipMemset failed");
         api_->device_synchronize();
     }
     return queue_counters_;

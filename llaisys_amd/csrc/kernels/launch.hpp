@@ -119,6 +119,7 @@ struct PagedAttentionPlan {
     int block_units_padded; // rounded up to a multiple of the XCD count
     int max_splits;      // split-KV partitions per unit
     int pages_per_split;
+    int pages_per_split_min; // the persistent kernel may cut splits down to this
     size_t partial_bytes; // workspace for split records
 };
 PagedAttentionPlan planPrefill(int B, int T, int nkvh, int group, int max_pages);
@@ -128,9 +129,11 @@ PagedAttentionPlan planPrefill(int B, int T, int nkvh, int group, int max_pages)
 // caller runs no pagedDecode for them.
 bool prefillQueueUsable(int B, const PagedAttentionPlan &plan, const int *queue);
 bool prefillTakesDecode(int B, int T, const PagedAttentionPlan &plan, const int *queue);
-// queue: two zeroed int32 counters that persist between calls (the
-// persistent kernel's work queue, left zero when it ends), or null for one
-// workgroup per (block, split) slot.
+// queue: kPrefillQueueWords zeroed int32 words that persist between calls:
+// the persistent kernel's two work-queue counters, left zero when it ends,
+// and last the split size it chose; or null for one workgroup per (block,
+// split) slot.
+constexpr int kPrefillQueueWords = 33;
 void pagedPrefill(void *out, bool out_f32, const uint16_t *q, const uint16_t *k_pool, const uint16_t *v_pool,
                   const int32_t *block_table, const int32_t *ctx_len, const int32_t *cu_q, int B, int T, int nh,
                   int nkvh, int max_pages, int num_blocks, float scale, const PagedAttentionPlan &plan,

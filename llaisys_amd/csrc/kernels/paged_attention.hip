@@ -34,6 +34,7 @@
 #include <algorithm>
 #include <cstdlib>
 #include <mutex>
+#include <type_traits>
 #include <vector>
 
 namespace llaisys::kernels {
@@ -48,6 +49,8 @@ constexpr int kWaves = 8;                                    // waves (groups) p
 constexpr int kStagePairs = 2;                               // page pairs per LDS stage (one barrier each)
 constexpr int kRecordFloats = kTiles * 16 * (kHeadDim + 2); // O for the group's columns, then (m, l)
 
+constexpr int kQueueSplitWord = kPrefillQueueWords - 1; // a cache line past the counters
+
 struct Args {
     const uint16_t *q;
     void *out;
@@ -58,7 +61,9 @@ struct Args {
     const int32_t *cu_q;
     float *records;
     int *err;
-    int *queue; // prefillQueueKernel: {next item, workgroups done}, zero between launches
+    int *queue; // prefillQueueKernel: {next item, workgroups done}, zero between launches; [kQueueSplitWord]: the split size it chose
+    int pps_min; // prefillQueueKernel may cut splits down to this many pages (pps: the most)
+    int cus;
     int with_decode; // pagedPrefill runs prefillQueueKernel<, true>: the single-query sequences too
     int B, T, nh, nkvh, G, max_pages, num_blocks, pps, max_splits, units, block_units, block_units_padded;
     float scale_log2;
@@ -96,6 +101,13 @@ __device__ bool locate(const Args &a, int index, bool blocks, int &b, int &local
     return false;
 }
 
+// Records of a unit: the splits of a table full of pages. CHOOSE: the
+// persistent kernel picks the split size (else a.pps). Instances of their own:
+// the choice in the plain ones moved their registers (2 us of the mixed step).
+template <bool CHOOSE> __device__ __forceinline__ int splitStride(const Args &a, int pps) {
+    return CHOOSE ? (a.max_pages + pps - 1) / pps : a.max_splits;
+}
+
 // Per-unit geometry shared by the attention and combine kernels. The visible
 // pages are those of the last query of the group's block, the same for every
 // group of a workgroup (their splits line up).
@@ -103,7 +115,7 @@ struct TileGeom {
     int b, group, q0, Lq, ctx, npages, nsplit;
 };
 
-__device__ bool blockGeom(const Args &a, int b, int block, TileGeom &t, bool report) {
+__device__ bool blockGeom(const Args &a, int b, int block, int pps, TileGeom &t, bool report) {
     t.b = b;
     t.q0 = a.cu_q[b];
     t.Lq = a.cu_q[b + 1] - t.q0;
@@ -115,7 +127,7 @@ __device__ bool blockGeom(const Args &a, int b, int block, TileGeom &t, bool rep
     const int qi_max = min(t.Lq - 1, ((block + 1) * kWaves * kTiles * 16 - 1) / a.G);
     const int kv_len = t.ctx - t.Lq + qi_max + 1; // keys some column of the block sees
     t.npages = (kv_len + 15) >> 4;
-    t.nsplit = (t.npages + a.pps - 1) / a.pps;
+    t.nsplit = (t.npages + pps - 1) / pps;
     return true;
 }
 
@@ -124,6 +136,8 @@ __device__ bool blockGeom(const Args &a, int b, int block, TileGeom &t, bool rep
 // the output's own, and it halves the record bytes that the attention kernel
 // writes and the combine reads. fp32 outputs keep fp32 records. The (m, l)
 // pairs stay fp32 after the O block either way.
+// (Chosen splits, of batches that would have had one or few, keep fp32
+// records too.)
 template <bool OUT_F32> __device__ __forceinline__ void storeRecordO(float *rec, int idx, f32x4 v) {
     if constexpr (OUT_F32) {
         *reinterpret_cast<f32x4 *>(rec + idx) = v;
@@ -149,17 +163,17 @@ typedef u32x4 StageBuf[2][kStagePairs * 16 * 64]; // page pairs: K a, K b, V a, 
 // (groups block * kWaves .. + kWaves - 1 of its groups_b; group_base groups
 // before the sequence), pages [split * pps, ...) of its t.npages. Called by
 // every wave of the workgroup with the same arguments (it has barriers).
-template <bool OUT_F32>
+template <bool OUT_F32, bool CHOOSE>
 __device__ __forceinline__ void prefillItem(const Args &a, StageBuf &kvs, int b, int block, int group_base, int h,
-                                            int split, int groups_b, const TileGeom &t) {
+                                            int split, int pps, int groups_b, const TileGeom &t) {
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6); // uniform: scalar branches on it
     const int lane = threadIdx.x & 63;
     const int n = lane & 15;
     const int grp = lane >> 4;
     const int G = a.G;
-    const int p0 = split * a.pps;
+    const int p0 = split * pps;
     if (p0 >= t.npages) return;
-    const int p1 = min(t.npages, p0 + a.pps);
+    const int p1 = min(t.npages, p0 + pps);
     const int group = block * kWaves + wave;        // this wave's group in the sequence
     const bool active = group < groups_b;
 
@@ -330,7 +344,7 @@ __device__ __forceinline__ void prefillItem(const Args &a, StageBuf &kvs, int b,
     if (bad_block && lane == 0) atomicOr(a.err, kErrBadBlock);
     if (!active) return;
     const int unit = (group_base + group) * a.nkvh + h;
-    float *rec = a.records + (size_t(unit) * a.max_splits + split) * kRecordFloats;
+    float *rec = a.records + (size_t(unit) * splitStride<CHOOSE>(a, pps) + split) * kRecordFloats;
 #pragma unroll
     for (int k = 0; k < kTiles; ++k) {
         float lt = acc[k].l + __shfl_xor(acc[k].l, 16);
@@ -345,7 +359,7 @@ __device__ __forceinline__ void prefillItem(const Args &a, StageBuf &kvs, int b,
         }
         const int c = k * 16 + n; // column within the group
 #pragma unroll
-        for (int i = 0; i < 8; ++i) storeRecordO<OUT_F32>(rec, (i * kTiles * 16 + c) * 16 + grp * 4, acc[k].o[i]);
+        for (int i = 0; i < 8; ++i) storeRecordO<OUT_F32 || CHOOSE>(rec, (i * kTiles * 16 + c) * 16 + grp * 4, acc[k].o[i]);
         if (grp == 0)
             *reinterpret_cast<float2 *>(rec + kTiles * 16 * kHeadDim + 2 * c) = make_float2(acc[k].m, lt);
     }
@@ -365,13 +379,14 @@ __global__ void __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_e
     block = __builtin_amdgcn_readfirstlane(block);
     group_base = __builtin_amdgcn_readfirstlane(group_base);
     TileGeom t;
-    if (!blockGeom(a, b, block, t, split == 0 && wave == 0)) return;
+    if (!blockGeom(a, b, block, a.pps, t, split == 0 && wave == 0)) return;
     // The geometry is wave-uniform: scalar registers, scalar branches.
     t.q0 = __builtin_amdgcn_readfirstlane(t.q0);
     t.Lq = __builtin_amdgcn_readfirstlane(t.Lq);
     t.ctx = __builtin_amdgcn_readfirstlane(t.ctx);
     t.npages = __builtin_amdgcn_readfirstlane(t.npages);
-    prefillItem<OUT_F32>(a, kvs, b, block, group_base, h, split, __builtin_amdgcn_readfirstlane(groupsOf(a, b)), t);
+    prefillItem<OUT_F32, false>(a, kvs, b, block, group_base, h, split, a.pps, __builtin_amdgcn_readfirstlane(groupsOf(a, b)),
+                         t);
 }
 
 // One single-query sequence's kv head h (query row `row`, c keys) in the
@@ -545,7 +560,7 @@ __host__ __device__ constexpr size_t queueTableInts(int B, int units) {
     return size_t(6) * (B + 1) + size_t(4) * (units + 1);
 }
 
-template <bool OUT_F32, bool WITH_DECODE>
+template <bool OUT_F32, bool WITH_DECODE, bool CHOOSE>
 __global__ void __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(2, 2)))
     prefillQueueKernel(Args a) {
     __shared__ StageBuf kvs;
@@ -624,9 +639,16 @@ __global__ void __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_e
         __syncthreads();
     }
     const int n_dec = n_dec_seqs * a.nkvh;
-    // Per unit: splits, full splits, partial flag.
+    // Per unit: its visible pages' splits, full splits and partial flag.
+    auto setSplits = [&](int u, int np, int pages) {
+        const int ns = (np + pages - 1) / pages;
+        const int full = np == ns * pages ? ns : ns - 1;
+        nspl[u] = ns;
+        fpre[u] = full;
+        ppos[u] = ns > full ? 1 : 0;
+    };
     for (int u = tid; u <= U; u += nthreads) {
-        int ns = 0, full = 0;
+        int np = 0;
         if (u < U) {
             const int b = lastAtMost(ubase, B, u);
             const int j = (u - ubase[b]) / a.nkvh;
@@ -635,16 +657,37 @@ __global__ void __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_e
                 if (blockIdx.x == 0 && u == ubase[b]) atomicOr(a.err, kErrTooLong);
             } else {
                 const int qi_max = min(lq - 1, ((j + 1) * kWaves * kTiles * 16 - 1) / a.G);
-                const int np = (c - lq + qi_max + 1 + 15) >> 4;
-                ns = (np + a.pps - 1) / a.pps;
-                full = np - (ns - 1) * a.pps == a.pps ? ns : ns - 1;
+                np = (c - lq + qi_max + 1 + 15) >> 4;
             }
         }
-        nspl[u] = ns;
-        fpre[u] = full;
-        ppos[u] = ns > full ? 1 : 0;
+        if constexpr (CHOOSE)
+            nspl[u] = np;
+        else
+            setSplits(u, np, a.pps);
     }
     __syncthreads();
+    // Pages per split: the fewest (a multiple of a stage, from pps_min) whose
+    // items still fit the CUs in one round, else pps. A split of 64 pages
+    // takes 45 us however few of them there are; finer ones than one round
+    // only add records (us with 64 pages / chosen, 12:2 heads: one prompt of
+    // 1000 tokens 44.5 / 34.6, of 2000 52.3 / 47.0, prompts of 350, 650 and
+    // 950 43.5 / 38.1, 64 tokens after 1000 46.2 / 27.9, 512 after 1500 48.0 /
+    // 38.0, six chunks of 100 after 2000 49.0 / 39.8).
+    // Every wave works it out by itself, from the coarsest down.
+    int pps = a.pps;
+    if constexpr (CHOOSE) {
+        for (int cand = pps - 2 * kStagePairs; cand >= a.pps_min; cand -= 2 * kStagePairs) {
+            const float inv = 1.f / float(cand);
+            int items = 0; // (rounding here moves a choice, not a result)
+            for (int u = tid & 63; u < U; u += 64) items += int(float(nspl[u] + cand - 1) * inv);
+            if (__builtin_amdgcn_readlane(waveInclusiveSum(items), 63) > a.cus) break;
+            pps = cand;
+        }
+        __syncthreads(); // every wave has read the page counts, which the splits replace
+        for (int u = tid; u <= U; u += nthreads) setSplits(u, nspl[u], pps);
+        if (blockIdx.x == 0 && tid == 0) a.queue[kQueueSplitWord] = pps;
+        __syncthreads();
+    }
     int n_full = 0, n_part = 0;
     blockExclusiveScan2(fpre, ppos, U + 1, scan_tmp, &n_full, &n_part);
     for (int u = tid; u < U; u += nthreads)
@@ -685,7 +728,7 @@ __global__ void __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_e
             t.nsplit = __builtin_amdgcn_readfirstlane(nspl[u]);
             const int group_base = __builtin_amdgcn_readfirstlane(gbase[b]);
             const int groups_b = __builtin_amdgcn_readfirstlane(gbase[b + 1]) - group_base;
-            prefillItem<OUT_F32>(a, kvs, b, block, group_base, h, split, groups_b, t);
+            prefillItem<OUT_F32, CHOOSE>(a, kvs, b, block, group_base, h, split, pps, groups_b, t);
         } else if constexpr (WITH_DECODE) {
             const int d = item - n_full;
             const int b = __builtin_amdgcn_readfirstlane(dseq[d / a.nkvh]);
@@ -703,7 +746,7 @@ __global__ void __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_e
 // Merge the split records of each unit with more than one split.
 constexpr int kMergeBatch = 4;
 
-template <bool OUT_F32> __global__ void __launch_bounds__(64) prefillCombineKernel(Args a) {
+template <bool OUT_F32, bool CHOOSE> __global__ void __launch_bounds__(64) prefillCombineKernel(Args a) {
     const int lane = threadIdx.x;
     const int n = lane & 15;
     const int grp = lane >> 4;
@@ -711,17 +754,27 @@ template <bool OUT_F32> __global__ void __launch_bounds__(64) prefillCombineKern
     const int k = blockIdx.x - unit * kTiles; // tile of the group this wave merges
     if (unit >= a.units) return;
     const int h = unit % a.nkvh;
+    // The split size prefillQueueKernel chose: requested here, by a vector
+    // load, beside the lengths that locate reads (a scalar load's wait would
+    // come before them), and needed after it.
+    int pps = a.pps;
+    if constexpr (CHOOSE) {
+        int at = kQueueSplitWord;
+        asm volatile("" : "+v"(at));
+        pps = a.queue[at];
+    }
     int b, group, group_base;
     if (!locate(a, unit / a.nkvh, false, b, group, group_base)) return;
+    pps = __builtin_amdgcn_readfirstlane(pps);
     TileGeom t;
-    if (!blockGeom(a, b, group / kWaves, t, false) || t.nsplit <= 1) return;
+    if (!blockGeom(a, b, group / kWaves, pps, t, false) || t.nsplit <= 1) return;
     const int G = a.G;
     const int pair = (group * kTiles + k) * 16 + n;
     const int qi = pair / G;
     const int g = pair - qi * G;
     const bool col_ok = qi < t.Lq;
     const int c = k * 16 + n;
-    const float *recs = a.records + size_t(unit) * a.max_splits * kRecordFloats;
+    const float *recs = a.records + size_t(unit) * splitStride<CHOOSE>(a, pps) * kRecordFloats;
     float M = -INFINITY, L = 0.f;
     f32x4 o[8];
 #pragma unroll
@@ -736,7 +789,7 @@ template <bool OUT_F32> __global__ void __launch_bounds__(64) prefillCombineKern
             mr[s] = k0 + s < t.nsplit ? ml.x : -INFINITY;
             lr[s] = ml.y;
 #pragma unroll
-            for (int i = 0; i < 8; ++i) orr[s][i] = loadRecordO<OUT_F32>(rec, (i * kTiles * 16 + c) * 16 + grp * 4);
+            for (int i = 0; i < 8; ++i) orr[s][i] = loadRecordO<OUT_F32 || CHOOSE>(rec, (i * kTiles * 16 + c) * 16 + grp * 4);
         }
 #pragma unroll
         for (int s = 0; s < kMergeBatch; ++s) {
@@ -792,7 +845,24 @@ PagedAttentionPlan planPrefill(int B, int T, int nkvh, int group, int max_pages)
     int pps = envInt("LLAISYS_PAGES_PER_SPLIT", 64);
     pps = std::max(2, std::min(128, pps & ~1));
     p.pages_per_split = pps;
-    p.max_splits = std::max(1, (max_pages + pps - 1) / pps);
+    // Batches whose blocks of queries leave CUs idle may take finer splits
+    // (down to 16 pages, chosen on the device, which knows the lengths), as
+    // far as 256 MiB of records go. Not where tables full of 64-page splits
+    // would give every CU one and a half: the choice is 64 there, and reading
+    // it back costs the merge a microsecond (the benchmark's mixed step 94.4
+    // us fixed, 95.6 chosen). Tables of up to 32 pages keep one split and no
+    // merge: at most 8 stages of a split, and the merge costs two.
+    p.pages_per_split_min = pps;
+    const long long blocks = ((long long)T * group + kWaves * kTiles * 16 - 1) / (kWaves * kTiles * 16) * nkvh;
+    if (!std::getenv("LLAISYS_PAGES_PER_SPLIT") && max_pages > 32 && blocks < cuCount() &&
+        blocks * max_pages < 96LL * cuCount()) {
+        constexpr size_t kMostBytes = size_t(256) << 20;
+        int least = 16;
+        while (least < pps && size_t(p.units) * ((max_pages + least - 1) / least) * kRecordFloats * sizeof(float) > kMostBytes)
+            least += 2 * kStagePairs;
+        p.pages_per_split_min = std::min(least, pps);
+    }
+    p.max_splits = std::max(1, (max_pages + p.pages_per_split_min - 1) / p.pages_per_split_min);
     p.partial_bytes = size_t(p.units) * p.max_splits * kRecordFloats * sizeof(float);
     return p;
 }
@@ -850,23 +920,27 @@ void pagedPrefill(void *out, bool out_f32, const uint16_t *q, const uint16_t *k_
     const size_t table_bytes = queueTableInts(B, plan.block_units) * sizeof(int);
     const bool queued = prefillQueueUsable(B, plan, queue);
     a.with_decode = queued && prefillTakesDecode(B, T, plan, queue);
+    a.pps_min = queued ? plan.pages_per_split_min : plan.pages_per_split;
+    a.cus = cuCount();
     const dim3 qgrid(unsigned(std::min<long long>(cuCount(), (long long)plan.block_units * plan.max_splits)));
+    const bool choose = a.pps_min < a.pps;
+    auto launch = [&](auto f32, auto chosen) {
+        constexpr bool F32 = decltype(f32)::value, CHOOSE = decltype(chosen)::value;
+        if (queued && a.with_decode)
+            hipLaunchKernelGGL((prefillQueueKernel<F32, true, CHOOSE>), qgrid, block, unsigned(table_bytes), s, a);
+        else if (queued)
+            hipLaunchKernelGGL((prefillQueueKernel<F32, false, CHOOSE>), qgrid, block, unsigned(table_bytes), s, a);
+        else
+            hipLaunchKernelGGL((prefillKernel<F32>), grid, block, 0, s, a);
+        if (plan.max_splits > 1)
+            hipLaunchKernelGGL((prefillCombineKernel<F32, CHOOSE>), dim3(plan.units * kTiles), cblock, 0, s, a);
+    };
     if (out_f32) {
-        if (queued && a.with_decode)
-            hipLaunchKernelGGL((prefillQueueKernel<true, true>), qgrid, block, unsigned(table_bytes), s, a);
-        else if (queued)
-            hipLaunchKernelGGL((prefillQueueKernel<true, false>), qgrid, block, unsigned(table_bytes), s, a);
-        else
-            hipLaunchKernelGGL((prefillKernel<true>), grid, block, 0, s, a);
-        if (plan.max_splits > 1) hipLaunchKernelGGL((prefillCombineKernel<true>), dim3(plan.units * kTiles), cblock, 0, s, a);
+        if (choose) launch(std::true_type(), std::true_type());
+        else launch(std::true_type(), std::false_type());
     } else {
-        if (queued && a.with_decode)
-            hipLaunchKernelGGL((prefillQueueKernel<false, true>), qgrid, block, unsigned(table_bytes), s, a);
-        else if (queued)
-            hipLaunchKernelGGL((prefillQueueKernel<false, false>), qgrid, block, unsigned(table_bytes), s, a);
-        else
-            hipLaunchKernelGGL((prefillKernel<false>), grid, block, 0, s, a);
-        if (plan.max_splits > 1) hipLaunchKernelGGL((prefillCombineKernel<false>), dim3(plan.units * kTiles), cblock, 0, s, a);
+        if (choose) launch(std::false_type(), std::true_type());
+        else launch(std::false_type(), std::false_type());
     }
     HIP_CHECK(hipGetLastError());
 }
