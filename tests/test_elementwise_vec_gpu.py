@@ -38,7 +38,8 @@ def test_add_and_swiglu(n, off, dtype):
 
 @pytest.mark.parametrize("dtype", list(TYPES))
 @pytest.mark.parametrize("rows,d", [(1, 1), (3, 7), (5, 8), (2, 520), (9, 1536), (4, 2048), (3, 2052), (2, 4096),
-                                    (2, 4104), (1, 10000)])
+                                    (2, 4104), (1, 10000), (1025, 8), (1027, 7),
+                                    (1026, 520), (1030, 1536), (1025, 2052), (1026, 4096), (1025, 4104)])
 @pytest.mark.parametrize("off", [0, 1])
 def test_rms_norm(rows, d, off, dtype):
     x, w = rnd((rows, d), dtype, 3), rnd((d,), dtype, 4)
