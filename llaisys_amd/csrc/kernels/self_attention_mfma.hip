@@ -28,7 +28,11 @@
 // product are then every fourth dim).
 //
 // 32-bit weights: P enters the 16-bit product as hi + lo (two MFMAs), f32
-// runs on the f32 MFMA.
+// runs on the f32 MFMA. Two halves hold a weight to 2^-17 or better as long
+// as neither leaves the type's range: always for bf16; f16 takes weights
+// below 2^-15 of a column's largest in passes of their own, scaled up (a
+// weight below 2^-25 is nothing in f16, and thousands of them can outweigh
+// the rest where their values are large).
 //
 // A weight of zero times a non-finite V is NaN, and a column must not see
 // keys past its own: a tile whose result is not finite is worked out again
@@ -146,7 +150,7 @@ __device__ __forceinline__ void columnByKeys(const T *qr, const T *k, const T *v
 template <typename T, int D, int CT, int WC, int WK, int KU>
 __global__ void __launch_bounds__(64 * WC * WK) selfAttentionMfmaKernel(AttnArgs a) {
     constexpr int ES = sizeof(T), NW = WC * WK;
-    constexpr bool F32 = ES == 4;
+    constexpr bool F32 = ES == 4, F16 = std::is_same<T, _Float16>::value;
     constexpr int PPR = D * ES / 16;        // 16 B pieces of a row
     constexpr int KW = 32 * KU;             // keys of a wave and stage
     constexpr int KS = KW * WK;             // keys of a stage
@@ -267,7 +271,9 @@ __global__ void __launch_bounds__(64 * WC * WK) selfAttentionMfmaKernel(AttnArgs
     };
     // The scores' weights in their place: online softmax in base 2, per
     // column. The running max moves (and O and l are rescaled) only when a column's
-    // scores exceed it by more than 2^8; the normalised result is the same.
+    // scores exceed it by more than 2^8; the normalised result is the same. f16:
+    // 2^7 higher, weights up to 2^15, which leaves the type's range to the small ones.
+    constexpr float kUp = F16 ? 7.f : 0.f;
     auto softmax = [&](f32x4 (&sc)[2 * KU][CT]) {
 #pragma unroll
         for (int ct = 0; ct < CT; ++ct) {
@@ -276,7 +282,7 @@ __global__ void __launch_bounds__(64 * WC * WK) selfAttentionMfmaKernel(AttnArgs
             for (int kt = 0; kt < 2 * KU; ++kt)
 #pragma unroll
                 for (int i = 0; i < 4; ++i) mx = fmaxf(mx, sc[kt][ct][i]);
-            mx = maxOverGroups(mx) * a.scale_log2; // (the scale is positive)
+            mx = maxOverGroups(mx) * a.scale_log2 - kUp; // (the scale is positive)
             const float m_true = fmaxf(m[ct], mx);
             if (__builtin_amdgcn_ballot_w64(m_true > m[ct] + 8.f) != 0) {
                 const float alpha = __builtin_amdgcn_exp2f(m[ct] - (m_true == -INFINITY ? 0.f : m_true));
@@ -319,37 +325,56 @@ __global__ void __launch_bounds__(64 * WC * WK) selfAttentionMfmaKernel(AttnArgs
             const int r = 4 * grp + (n >> 2); // the lane's row of a 16-key V read
             const uint32_t vbase = uint32_t(uintptr_t((lds_void *)vs)) + 16 * PPR * r + 8 * (n & 1);
             const int half = (n >> 1) & 1;
+            // One pass: the weights that are at least kSmall when scaled by `up`
+            // (a power of two; bf16: all of them); whether a lane has smaller ones.
+            constexpr float kSmall = 0x1p-8f, kStep = 0x1p23f;
+            auto pass = [&](auto first, float up) {
+                constexpr bool FIRST = decltype(first)::value;
+                bool rest = false;
 #pragma unroll
-            for (int u = 0; u < KU; ++u) {
-                typename P::type hi[CT], lo[CT];
+                for (int u = 0; u < KU; ++u) {
+                    typename P::type hi[CT], lo[CT];
 #pragma unroll
-                for (int ct = 0; ct < CT; ++ct)
+                    for (int ct = 0; ct < CT; ++ct)
 #pragma unroll
-                    for (int e = 0; e < 8; ++e) {
-                        const float p = sc[2 * u + (e >> 2)][ct][e & 3];
-                        hi[ct][e] = T(p);
-                        lo[ct][e] = T(p - float(hi[ct][e]));
-                    }
+                        for (int e = 0; e < 8; ++e) {
+                            float p = sc[2 * u + (e >> 2)][ct][e & 3];
+                            if constexpr (F16) {
+                                if (!FIRST) p = p * up < kSmall * kStep ? p * up : 0.f;
+                                rest |= p > 0.f && p < kSmall;
+                                p = p < kSmall ? 0.f : p;
+                            }
+                            hi[ct][e] = T(p);
+                            lo[ct][e] = T(p - float(hi[ct][e]));
+                        }
 #pragma unroll
-                for (int i0 = 0; i0 < D / 16; i0 += 4) {
-                    uint32_t at[4];
+                    for (int i0 = 0; i0 < D / 16; i0 += 4) {
+                        uint32_t at[4];
 #pragma unroll
-                    for (int i = 0; i < 4; ++i)
-                        at[i] = vbase + u * 32 * PPR * 16 + 16 * ((2 * (i0 + i) + half) ^ rowKey<PPR>(r));
-                    u32x2 w[8];
-                    readV4<16 * PPR * 16>(w, at);
+                        for (int i = 0; i < 4; ++i)
+                            at[i] = vbase + u * 32 * PPR * 16 + 16 * ((2 * (i0 + i) + half) ^ rowKey<PPR>(r));
+                        u32x2 w[8];
+                        readV4<16 * PPR * 16>(w, at);
 #pragma unroll
-                    for (int i = 0; i < 4; ++i) {
-                        const auto vf = __builtin_bit_cast(
-                            typename P::type, u32x4{w[2 * i][0], w[2 * i][1], w[2 * i + 1][0], w[2 * i + 1][1]});
+                        for (int i = 0; i < 4; ++i) {
+                            const auto vf = __builtin_bit_cast(
+                                typename P::type, u32x4{w[2 * i][0], w[2 * i][1], w[2 * i + 1][0], w[2 * i + 1][1]});
 #pragma unroll
-                        for (int ct = 0; ct < CT; ++ct) {
-                            acc[ct][i0 + i] = P::mfma(vf, hi[ct], acc[ct][i0 + i]);
-                            acc[ct][i0 + i] = P::mfma(vf, lo[ct], acc[ct][i0 + i]);
+                            for (int ct = 0; ct < CT; ++ct) {
+                                f32x4 &o = acc[ct][i0 + i];
+                                if constexpr (FIRST)
+                                    o = P::mfma(vf, lo[ct], P::mfma(vf, hi[ct], o));
+                                else
+                                    o += P::mfma(vf, lo[ct], P::mfma(vf, hi[ct], f32x4{0.f, 0.f, 0.f, 0.f})) * (1.f / up);
+                            }
                         }
                     }
                 }
-            }
+                return __builtin_amdgcn_ballot_w64(rest) != 0;
+            };
+            bool rest = pass(std::true_type(), 1.f);
+            if constexpr (F16)
+                for (float up = kStep; rest && up < INFINITY; up *= kStep) rest = pass(std::false_type(), up);
         }
     };
 

@@ -102,6 +102,27 @@ def test_values_past_a_query_do_not_reach_it(Lq, S, dtype):
         assert torch.isnan(got[-1]).all()
 
 
+# One key takes nearly all the weight and has a small value; 4000 others have
+# 2^-gap of its weight each and values of 30000. Nothing of the sum may be lost
+# to the range of the 16-bit type: dim 0 is their sum, dim 1 the large weight's
+# own value. (S = 4001; L = 40 also runs tiles of more columns.)
+@pytest.mark.parametrize("dtype", list(TYPES))
+@pytest.mark.parametrize("gap", [14.0, 17.5, 26.5, 34.0, 45.0, 70.0])
+@pytest.mark.parametrize("Lq,d", [(1, 64), (40, 128)])
+def test_small_weights_of_large_values(Lq, d, gap, dtype):
+    t = TYPES[dtype]
+    q = torch.zeros(Lq, 12, d, device="cuda", dtype=t)
+    k, v = torch.zeros(4000 + Lq, 2, d, device="cuda", dtype=t), torch.zeros(4000 + Lq, 2, d, device="cuda", dtype=t)
+    q[..., 0], k[1000, :, 0] = 8.0, gap / 8
+    v[..., 0], v[1000, :, 0], v[1000, :, 1] = 30000.0, 0.0, 1.0
+    scale = float(math.log(2.0))  # scores in powers of two
+    got, want = run(q, k, v, scale), exact(q, k, v, scale)
+    half_ulp = {torch.float32: 2.0**-24, torch.float16: 2.0**-11, torch.bfloat16: 2.0**-8}[t]
+    # weights to 2^-16 of their own size; gap ulps of the exponent (|s| 2^-24, twice); f16's least step
+    rel = half_ulp + (2.0**-16 if t != torch.float32 else 2.0**-18) + gap * 2.0**-23
+    assert torch.all((got.double() - want).abs() <= rel * want.abs() + (2.0**-25 if t == torch.float16 else 0.0))
+
+
 def test_infinite_value_that_is_seen():
     q, k, v = inputs(9, 300, 12, 2, 128, torch.bfloat16)
     v[5, 0, 7] = math.inf
