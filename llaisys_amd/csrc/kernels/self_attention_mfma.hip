@@ -32,7 +32,14 @@
 // as neither leaves the type's range: always for bf16; f16 takes weights
 // below 2^-15 of a column's largest in passes of their own, scaled up (a
 // weight below 2^-25 is nothing in f16, and thousands of them can outweigh
-// the rest where their values are large).
+// the rest where their values are large). What that takes where no weight is
+// small: 1000 x 1000 19.5 -> 20.4 us, 512 x 1536 17.4 -> 19.2.
+//
+// The f32 MFMAs add their four products to one running sum, so a long chain
+// of them rounds as often as it is long. The scores take four chains and the
+// values a fresh one every stage: error against 64 bits (2-norm) at 512 x 1536
+// 5.2e-7 -> 2.2e-7, 1 x 513 4.2e-7 -> 2.2e-7 (4.3e-7 and 4.0e-7 by plain FMAs),
+// for 65.1 us instead of 60.5 and 10.0 instead of 9.7.
 //
 // A weight of zero times a non-finite V is NaN, and a column must not see
 // keys past its own: a tile whose result is not finite is worked out again
@@ -231,10 +238,14 @@ __global__ void __launch_bounds__(64 * WC * WK) selfAttentionMfmaKernel(AttnArgs
 
     // S^T of the wave's keys from LDS, those a column may not see at -inf.
     auto scores = [&](const u32x4 *ks, int key0, f32x4 (&sc)[2 * KU][CT]) {
+        constexpr int CH = F32 ? 4 : 1; // chains of a sum
+        f32x4 part[CH][2 * KU][CT];
 #pragma unroll
-        for (int kt = 0; kt < 2 * KU; ++kt)
+        for (int e = 0; e < CH; ++e)
 #pragma unroll
-            for (int ct = 0; ct < CT; ++ct) sc[kt][ct] = f32x4{0.f, 0.f, 0.f, 0.f};
+            for (int kt = 0; kt < 2 * KU; ++kt)
+#pragma unroll
+                for (int ct = 0; ct < CT; ++ct) part[e][kt][ct] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int s = 0; s < (F32 ? D / 16 : D / 32); ++s) {
             u32x4 kf[2 * KU];
@@ -247,18 +258,25 @@ __global__ void __launch_bounds__(64 * WC * WK) selfAttentionMfmaKernel(AttnArgs
                     for (int kt = 0; kt < 2 * KU; ++kt)
 #pragma unroll
                         for (int ct = 0; ct < CT; ++ct)
-                            sc[kt][ct] = __builtin_amdgcn_mfma_f32_16x16x4f32(
-                                __uint_as_float(kf[kt][e]), __uint_as_float(qop[ct][s][e]), sc[kt][ct], 0, 0, 0);
+                            part[e][kt][ct] = __builtin_amdgcn_mfma_f32_16x16x4f32(
+                                __uint_as_float(kf[kt][e]), __uint_as_float(qop[ct][s][e]), part[e][kt][ct], 0, 0, 0);
             } else {
                 using P = Piece<T>;
 #pragma unroll
                 for (int kt = 0; kt < 2 * KU; ++kt)
 #pragma unroll
                     for (int ct = 0; ct < CT; ++ct)
-                        sc[kt][ct] = P::mfma(__builtin_bit_cast(typename P::type, kf[kt]),
-                                             __builtin_bit_cast(typename P::type, qop[ct][s]), sc[kt][ct]);
+                        part[0][kt][ct] = P::mfma(__builtin_bit_cast(typename P::type, kf[kt]),
+                                                  __builtin_bit_cast(typename P::type, qop[ct][s]), part[0][kt][ct]);
             }
         }
+#pragma unroll
+        for (int kt = 0; kt < 2 * KU; ++kt)
+#pragma unroll
+            for (int ct = 0; ct < CT; ++ct) {
+                sc[kt][ct] = part[0][kt][ct];
+                if constexpr (F32) sc[kt][ct] = (sc[kt][ct] + part[1][kt][ct]) + (part[2][kt][ct] + part[3][kt][ct]);
+            }
         if (key0 + KW - 1 > lim_lo) {
 #pragma unroll
             for (int kt = 0; kt < 2 * KU; ++kt)
@@ -306,20 +324,30 @@ __global__ void __launch_bounds__(64 * WC * WK) selfAttentionMfmaKernel(AttnArgs
     auto addValues = [&](const u32x4 *vs, const f32x4 (&sc)[2 * KU][CT]) {
         if constexpr (F32) {
 #pragma unroll
-            for (int kt = 0; kt < 2 * KU; ++kt)
+            for (int b = 0; b < D / 64; ++b) {
+                f32x4 sum[4][CT];
 #pragma unroll
-                for (int i = 0; i < 4; ++i)
+                for (int j = 0; j < 4; ++j)
 #pragma unroll
-                    for (int b = 0; b < D / 64; ++b) {
+                    for (int ct = 0; ct < CT; ++ct) sum[j][ct] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int kt = 0; kt < 2 * KU; ++kt)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
                         const int r = kt * 16 + 4 * grp + i;
                         const u32x4 vf = vs[r * PPR + ((16 * b + n) ^ rowKey<PPR>(r))];
 #pragma unroll
                         for (int j = 0; j < 4; ++j)
 #pragma unroll
                             for (int ct = 0; ct < CT; ++ct)
-                                acc[ct][4 * b + j] = __builtin_amdgcn_mfma_f32_16x16x4f32(
-                                    __uint_as_float(vf[j]), sc[kt][ct][i], acc[ct][4 * b + j], 0, 0, 0);
+                                sum[j][ct] = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(vf[j]), sc[kt][ct][i],
+                                                                                  sum[j][ct], 0, 0, 0);
                     }
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+#pragma unroll
+                    for (int ct = 0; ct < CT; ++ct) acc[ct][4 * b + j] += sum[j][ct];
+            }
         } else {
             using P = Piece<T>;
             const int r = 4 * grp + (n >> 2); // the lane's row of a 16-key V read
