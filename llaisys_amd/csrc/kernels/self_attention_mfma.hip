@@ -42,8 +42,13 @@
 // for 65.1 us instead of 60.5 and 10.0 instead of 9.7.
 //
 // A weight of zero times a non-finite V is NaN, and a column must not see
-// keys past its own: a tile whose result is not finite is worked out again
-// column by column over the keys it may see, in plain FMAs.
+// keys past its own; nor may the lazy max's larger weights overflow a sum. A
+// tile whose result is not finite is worked out again with weights of at most
+// one: rows of V that hold a huge value are zeros to the MFMAs and go to the
+// columns that see them in plain FMAs, and only the columns in question are
+// written. An inf in the first of 1000 x 1000 keys: 46 us (those columns one
+// by one over their keys: 670, and the general kernel 490); 1 x 513: 21 us
+// (92, and 15).
 #include "lanes.hpp"
 #include "launch.hpp"
 #include "self_attention.hpp"
@@ -118,40 +123,20 @@ template <int NEXT> __device__ __forceinline__ void readV4(u32x2 (&w)[8], const 
 
 __device__ __forceinline__ bool finite(float x) { return __builtin_fabsf(x) <= 3.402823466e38f; }
 
-// One column over keys [k0, k1) by one wave in plain FMAs: m, l, and o of
-// dims lane, lane + 64, ...
-template <typename T, int D>
-__device__ __forceinline__ void columnByKeys(const T *qr, const T *k, const T *v, size_t stride, int k0, int k1,
-                                          float scale_log2, float &m, float &l, float (&o)[D / 64]) {
-    const int lane = threadIdx.x & 63;
-    m = -INFINITY;
-    l = 0.f;
-    for (int c = 0; c < D / 64; ++c) o[c] = 0.f;
-    for (int j0 = k0; j0 < k1; j0 += 64) {
-        const int j = j0 + lane;
-        float s = -INFINITY;
-        if (j < k1) {
-            float dot = 0.f;
-            for (int e = 0; e < D; ++e) dot = fmaf(float(qr[e]), float(k[size_t(j) * stride + e]), dot);
-            s = dot * scale_log2;
-        }
-        float mx = s;
-        for (int off = 32; off > 0; off >>= 1) mx = fmaxf(mx, __shfl_xor(mx, off));
-        const float m_new = fmaxf(m, mx);
-        const float alpha = exp2f(m - m_new);
-        const float p = j < k1 ? exp2f(s - m_new) : 0.f;
-        float ps = p;
-        for (int off = 32; off > 0; off >>= 1) ps += __shfl_xor(ps, off);
-        l = l * alpha + ps;
-        m = m_new;
-        for (int c = 0; c < D / 64; ++c) o[c] *= alpha;
-        const int cnt = min(64, k1 - j0);
-        for (int u = 0; u < cnt; ++u) {
-            const float pu = __shfl(p, u);
-            for (int c = 0; c < D / 64; ++c)
-                o[c] = fmaf(pu, float(v[size_t(j0 + u) * stride + lane + 64 * c]), o[c]);
+// Whether a 16 B piece of V holds a value whose products could leave the range
+// of the sums: inf, NaN, and of the types with f32's exponents 2^100 and more.
+template <typename T> __device__ __forceinline__ bool holdsHuge(const u32x4 &w) {
+    bool huge = false;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        if constexpr (sizeof(T) == 4) {
+            huge |= (w[e] & 0x7fffffffu) >= 0x71800000u;
+        } else {
+            constexpr uint32_t kFrom = std::is_same<T, _Float16>::value ? 0x7c00u : 0x7180u;
+            huge |= (w[e] & 0x7fffu) >= kFrom || ((w[e] >> 16) & 0x7fffu) >= kFrom;
         }
     }
+    return huge;
 }
 
 template <typename T, int D, int CT, int WC, int WK, int KU>
@@ -170,7 +155,7 @@ __global__ void __launch_bounds__(64 * WC * WK) selfAttentionMfmaKernel(AttnArgs
     extern __shared__ u32x4 lds[]; // NB stages; afterwards the waves' partial states
     __shared__ int bad[COLS];
 
-    const int lane = threadIdx.x & 63, n = lane & 15, grp = lane >> 4;
+    int lane = threadIdx.x & 63, n = lane & 15, grp = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int wc = wave % WC, wk = wave / WC;
     // Tiles from the last (most keys) to the first; neighbouring workgroups
@@ -289,10 +274,10 @@ __global__ void __launch_bounds__(64 * WC * WK) selfAttentionMfmaKernel(AttnArgs
     };
     // The scores' weights in their place: online softmax in base 2, per
     // column. The running max moves (and O and l are rescaled) only when a column's
-    // scores exceed it by more than 2^8; the normalised result is the same. f16:
+    // scores exceed it by more than 2^lazy; the normalised result is the same. f16:
     // 2^7 higher, weights up to 2^15, which leaves the type's range to the small ones.
-    constexpr float kUp = F16 ? 7.f : 0.f;
-    auto softmax = [&](f32x4 (&sc)[2 * KU][CT]) {
+    constexpr float kLazy = 8.f, kUp = F16 ? 7.f : 0.f;
+    auto softmax = [&](f32x4 (&sc)[2 * KU][CT], float lazy) {
 #pragma unroll
         for (int ct = 0; ct < CT; ++ct) {
             float mx = sc[0][ct][0];
@@ -302,7 +287,7 @@ __global__ void __launch_bounds__(64 * WC * WK) selfAttentionMfmaKernel(AttnArgs
                 for (int i = 0; i < 4; ++i) mx = fmaxf(mx, sc[kt][ct][i]);
             mx = maxOverGroups(mx) * a.scale_log2 - kUp; // (the scale is positive)
             const float m_true = fmaxf(m[ct], mx);
-            if (__builtin_amdgcn_ballot_w64(m_true > m[ct] + 8.f) != 0) {
+            if (__builtin_amdgcn_ballot_w64(m_true > m[ct] + lazy) != 0) {
                 const float alpha = __builtin_amdgcn_exp2f(m[ct] - (m_true == -INFINITY ? 0.f : m_true));
                 l[ct] *= alpha;
 #pragma unroll
@@ -406,142 +391,200 @@ __global__ void __launch_bounds__(64 * WC * WK) selfAttentionMfmaKernel(AttnArgs
         }
     };
 
-    if constexpr (PRIV) {
-        // One column group: a wave shares its keys with no other, so each runs
-        // its own pair of buffers without barriers: the next keys' K is on its
-        // way while the weights and the values of these are worked out, their
-        // V during the next scores. (Past the end rows of zeros, or unused.)
-        u32x4 *kb = lds + 2 * wave * KW * PPR, *vb = kb + KW * PPR;
-        constexpr int LW = KW / RPI;
-        const std::integral_constant<int, 1> one;
-        const std::integral_constant<int, LW> lw;
-        auto issue = [&](const __amdgpu_buffer_rsrc_t &rsrc, u32x4 *dst, int st) {
-            load(rsrc, dst - wk * KW * PPR, st, wk * LW, one, lw);
-        };
-        const int n_st = min(s1, lim_hi < wk * KW ? 0 : (lim_hi - wk * KW) / KS + 1); // the wave's last stage + 1
-        if (s0 < n_st) {
-            issue(kr, kb, s0);
-            issue(vr, vb, s0);
-        }
-        for (int st = s0; st < n_st; ++st) {
-            f32x4 sc[2 * KU][CT];
-            asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LW) : "memory");
-            scores(kb, st * KS + wk * KW, sc);
-            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-            issue(kr, kb, st + 1);
-            softmax(sc);
-            asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LW) : "memory");
-            addValues(vb, sc);
-            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-            issue(vr, vb, st + 1);
-        }
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    } else {
-        const std::integral_constant<int, NW> step;
-        const std::integral_constant<int, KS / RPI / NW> count;
-        auto issue = [&](int st, int buf) {
-            load(kr, lds + buf * STAGE, st, wave, step, count);
-            load(vr, lds + buf * STAGE + KS * PPR, st, wave, step, count);
-        };
-        if (s0 < s1) issue(s0, 0);
-        for (int st = s0; st < s1; ++st) {
-            const int buf = (st - s0) & 1;
-            // This stage has landed, and everyone has read the one whose buffer the next takes.
-            asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-            if (st + 1 < s1) issue(st + 1, buf ^ 1);
-            const int key0 = st * KS + wk * KW;
-            if (key0 > lim_hi) continue; // none of the wave's columns sees these keys
-            const u32x4 *ks = lds + buf * STAGE + wk * KW * PPR;
-            f32x4 sc[2 * KU][CT];
-            scores(ks, key0, sc);
-            softmax(sc);
-            addValues(ks + KS * PPR, sc);
-        }
-    }
-
-    // The waves' states into LDS (every stage has been read), column-major.
-    float *po = reinterpret_cast<float *>(lds), *pml = po + NW * CT * 16 * OP;
-    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-#pragma unroll
-    for (int ct = 0; ct < CT; ++ct) {
-        const float lt = sumOverGroups(l[ct]);
-        const int c = (wave * CT + ct) * 16 + n;
-        if (grp == 0) *reinterpret_cast<f32x2 *>(pml + 2 * c) = f32x2{m[ct], lt};
-#pragma unroll
-        for (int i = 0; i < D / 16; ++i) {
-            if constexpr (F32) {
-                const int b = i / 4, e = i % 4;
-                *reinterpret_cast<f32x4 *>(po + c * OP + 64 * b + 16 * grp + 4 * e) =
-                    f32x4{acc[ct][4 * b][e], acc[ct][4 * b + 1][e], acc[ct][4 * b + 2][e], acc[ct][4 * b + 3][e]};
-            } else {
-                *reinterpret_cast<f32x4 *>(po + c * OP + 16 * i + 4 * grp) = acc[ct][i];
+    // The scores, weights and values of stages [s0, s1).
+    auto run = [&]() {
+        if constexpr (PRIV) {
+            // One column group: a wave shares its keys with no other, so each runs
+            // its own pair of buffers without barriers: the next keys' K is on its
+            // way while the weights and the values of these are worked out, their
+            // V during the next scores. (Past the end rows of zeros, or unused.)
+            u32x4 *kb = lds + 2 * wave * KW * PPR, *vb = kb + KW * PPR;
+            constexpr int LW = KW / RPI;
+            const std::integral_constant<int, 1> one;
+            const std::integral_constant<int, LW> lw;
+            auto issue = [&](const __amdgpu_buffer_rsrc_t &rsrc, u32x4 *dst, int st) {
+                load(rsrc, dst - wk * KW * PPR, st, wk * LW, one, lw);
+            };
+            const int n_st = min(s1, lim_hi < wk * KW ? 0 : (lim_hi - wk * KW) / KS + 1); // the wave's last stage + 1
+            if (s0 < n_st) {
+                issue(kr, kb, s0);
+                issue(vr, vb, s0);
+            }
+            for (int st = s0; st < n_st; ++st) {
+                f32x4 sc[2 * KU][CT];
+                asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LW) : "memory");
+                scores(kb, st * KS + wk * KW, sc);
+                asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+                issue(kr, kb, st + 1);
+                softmax(sc, kLazy);
+                asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LW) : "memory");
+                addValues(vb, sc);
+                asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+                issue(vr, vb, st + 1);
+            }
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        } else {
+            const std::integral_constant<int, NW> step;
+            const std::integral_constant<int, KS / RPI / NW> count;
+            auto issue = [&](int st, int buf) {
+                load(kr, lds + buf * STAGE, st, wave, step, count);
+                load(vr, lds + buf * STAGE + KS * PPR, st, wave, step, count);
+            };
+            if (s0 < s1) issue(s0, 0);
+            for (int st = s0; st < s1; ++st) {
+                const int buf = (st - s0) & 1;
+                // This stage has landed, and everyone has read the one whose buffer the next takes.
+                asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+                if (st + 1 < s1) issue(st + 1, buf ^ 1);
+                const int key0 = st * KS + wk * KW;
+                if (key0 > lim_hi) continue; // none of the wave's columns sees these keys
+                const u32x4 *ks = lds + buf * STAGE + wk * KW * PPR;
+                f32x4 sc[2 * KU][CT];
+                scores(ks, key0, sc);
+                softmax(sc, kLazy);
+                addValues(ks + KS * PPR, sc);
             }
         }
-    }
-    for (int c = threadIdx.x; c < COLS; c += 64 * NW) bad[c] = 0;
-    __syncthreads();
-    // Column c's WK states are those of waves wc + WC k; 4 dims a thread.
-    auto put = [&](int c, int d0, f32x4 o, float M, float Ls) {
-        const int cc = col0 + c, qi = cc / a.G;
-        const size_t row = size_t(qi) * a.nh + kh * a.G + (cc - qi * a.G);
-        if (a.NS > 1) {
-            float *rec = a.part + (row * a.NS + z) * (D + 2);
-            if (d0 == 0) *reinterpret_cast<f32x2 *>(rec) = f32x2{M, Ls};
-            *reinterpret_cast<f32x2 *>(rec + 2 + d0) = f32x2{o[0], o[1]};
-            *reinterpret_cast<f32x2 *>(rec + 4 + d0) = f32x2{o[2], o[3]};
-            return;
-        }
-        typedef T t4 __attribute__((ext_vector_type(4)));
-        const float inv = 1.f / Ls;
-        *reinterpret_cast<t4 *>(static_cast<T *>(a.out) + row * D + d0) =
-            t4{T(o[0] * inv), T(o[1] * inv), T(o[2] * inv), T(o[3] * inv)};
     };
-    int any_bad = 0;
-    for (int i = threadIdx.x; i < COLS * (D / 4); i += 64 * NW) {
-        const int c = i / (D / 4), d0 = 4 * (i % (D / 4));
-        if (col0 + c >= cols) break;
-        const int w0 = c / (CT * 16), cl = c % (CT * 16);
-        float M = -INFINITY;
+    // The same with one buffer, weights of at most one and the huge rows apart.
+    auto runAgain = [&]() {
 #pragma unroll
-        for (int k = 0; k < WK; ++k) M = fmaxf(M, pml[2 * ((w0 + WC * k) * CT * 16 + cl)]);
-        float Ls = 0.f;
-        f32x4 o = {0.f, 0.f, 0.f, 0.f};
-        const float Mu = M == -INFINITY ? 0.f : M; // no key of this split seen: weights 0
+        for (int ct = 0; ct < CT; ++ct) {
+            m[ct] = -INFINITY;
+            l[ct] = 0.f;
 #pragma unroll
-        for (int k = 0; k < WK; ++k) {
-            const int x = (w0 + WC * k) * CT * 16 + cl;
-            const float w = __builtin_amdgcn_exp2f(pml[2 * x] - Mu);
-            Ls += pml[2 * x + 1] * w;
-            o += *reinterpret_cast<const f32x4 *>(po + x * OP + d0) * w;
+            for (int i = 0; i < D / 16; ++i) acc[ct][i] = f32x4{0.f, 0.f, 0.f, 0.f};
         }
-        const bool fine = finite(o[0]) && finite(o[1]) && finite(o[2]) && finite(o[3]) && finite(Ls);
-        if (!fine) {
-            bad[c] = 1;
-            any_bad = 1;
+        const std::integral_constant<int, NW> step;
+        const std::integral_constant<int, KS / RPI / NW> count;
+        const u32x4 *ks = lds + wk * KW * PPR;
+        u32x4 *vs = lds + (KS + wk * KW) * PPR;
+        for (int st = s0; st < s1; ++st) {
+            __syncthreads(); // everyone has read the stage before
+            load(kr, lds, st, wave, step, count);
+            load(vr, lds + KS * PPR, st, wave, step, count);
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            __syncthreads();
+            uint64_t huge = 0; // of the wave's keys
+            for (int b = 0; b < KW / RPI; ++b) {
+                const uint64_t pieces = __builtin_amdgcn_ballot_w64(holdsHuge<T>(vs[b * 64 + lane]));
+                for (int r = 0; r < RPI; ++r)
+                    if ((pieces >> (r * PPR)) & ((1ull << PPR) - 1)) huge |= 1ull << (b * RPI + r);
+            }
+            __syncthreads(); // (the waves of other columns share these rows)
+            for (int b = 0; b < KW / RPI; ++b)
+                if ((huge >> (b * RPI + lane / PPR)) & 1) vs[b * 64 + lane] = u32x4{0, 0, 0, 0};
+            __syncthreads();
+            const int key0 = st * KS + wk * KW;
+            if (key0 > lim_hi) continue;
+            f32x4 sc[2 * KU][CT];
+            scores(ks, key0, sc);
+            softmax(sc, 0.f);
+            addValues(vs, sc);
+            for (; huge; huge &= huge - 1) {
+                const int j = __builtin_ctzll(huge), key = key0 + j;
+                const T *vrow = static_cast<const T *>(a.v) + (size_t(key) * a.nkvh + kh) * D;
+#pragma unroll
+                for (int ct = 0; ct < CT; ++ct) {
+                    // Key 16 kt + 4 g + i of the wave's is element i of lane group g.
+                    float p = 0.f;
+#pragma unroll
+                    for (int kt = 0; kt < 2 * KU; ++kt)
+#pragma unroll
+                        for (int i = 0; i < 4; ++i)
+                            if (j / 16 == kt && j % 4 == i) p = sc[kt][ct][i];
+                    p = __shfl(p, (j / 4 % 4) * 16 + n);
+#pragma unroll
+                    for (int i = 0; i < D / 16; ++i)
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) {
+                            const int dim = F32 ? 64 * (i / 4) + 16 * grp + 4 * e + i % 4 : 16 * i + 4 * grp + e;
+                            const float sum = fmaf(p, float(vrow[dim]), acc[ct][i][e]);
+                            acc[ct][i][e] = key <= limit[ct] ? sum : acc[ct][i][e];
+                            asm volatile("" ::: "memory"); // (a load at a time: registers)
+                        }
+                }
+            }
         }
-        put(c, d0, o, M, Ls);
-    }
-    if (!__syncthreads_or(any_bad)) return;
-    for (int c = wave; c < COLS && col0 + c < cols; c += NW) {
-        if (!bad[c]) continue;
-        const int cc = col0 + c, qi = cc / a.G;
-        const T *kb = static_cast<const T *>(a.k) + size_t(kh) * D, *vb = static_cast<const T *>(a.v) + size_t(kh) * D;
-        float M, Ls, o[D / 64];
-        columnByKeys<T, D>(qp + (size_t(qi) * a.nh + kh * a.G + (cc - qi * a.G)) * D, kb, vb, size_t(a.nkvh) * D,
-                           s0 * KS, min(s1 * KS, qi + shift + 1), a.scale_log2, M, Ls, o);
-        const size_t row = size_t(qi) * a.nh + kh * a.G + (cc - qi * a.G);
-        float *rec = a.part + (row * a.NS + z) * (D + 2);
-        if (a.NS > 1 && lane == 0) {
-            rec[0] = M;
-            rec[1] = Ls;
+    };
+
+    // The waves' states to the results; AGAIN: of the columns in bad, else
+    // filling bad. Whether some column is.
+    auto finish = [&](auto second) {
+        constexpr bool AGAIN = decltype(second)::value;
+        // The waves' states into LDS (every stage has been read), column-major.
+        float *po = reinterpret_cast<float *>(lds), *pml = po + NW * CT * 16 * OP;
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+#pragma unroll
+        for (int ct = 0; ct < CT; ++ct) {
+            const float lt = sumOverGroups(l[ct]);
+            const int c = (wave * CT + ct) * 16 + n;
+            if (grp == 0) *reinterpret_cast<f32x2 *>(pml + 2 * c) = f32x2{m[ct], lt};
+#pragma unroll
+            for (int i = 0; i < D / 16; ++i) {
+                if constexpr (F32) {
+                    const int b = i / 4, e = i % 4;
+                    *reinterpret_cast<f32x4 *>(po + c * OP + 64 * b + 16 * grp + 4 * e) =
+                        f32x4{acc[ct][4 * b][e], acc[ct][4 * b + 1][e], acc[ct][4 * b + 2][e], acc[ct][4 * b + 3][e]};
+                } else {
+                    *reinterpret_cast<f32x4 *>(po + c * OP + 16 * i + 4 * grp) = acc[ct][i];
+                }
+            }
         }
-        for (int i = 0; i < D / 64; ++i) {
-            if (a.NS > 1)
-                rec[2 + lane + 64 * i] = o[i];
-            else
-                static_cast<T *>(a.out)[row * D + lane + 64 * i] = T(o[i] / Ls);
+        if (!AGAIN)
+            for (int c = threadIdx.x; c < COLS; c += 64 * NW) bad[c] = 0;
+        __syncthreads();
+        // Column c's WK states are those of waves wc + WC k; 4 dims a thread.
+        auto put = [&](int c, int d0, f32x4 o, float M, float Ls) {
+            const int cc = col0 + c, qi = cc / a.G;
+            const size_t row = size_t(qi) * a.nh + kh * a.G + (cc - qi * a.G);
+            if (a.NS > 1) {
+                float *rec = a.part + (row * a.NS + z) * (D + 2);
+                if (d0 == 0) *reinterpret_cast<f32x2 *>(rec) = f32x2{M, Ls};
+                *reinterpret_cast<f32x2 *>(rec + 2 + d0) = f32x2{o[0], o[1]};
+                *reinterpret_cast<f32x2 *>(rec + 4 + d0) = f32x2{o[2], o[3]};
+                return;
+            }
+            typedef T t4 __attribute__((ext_vector_type(4)));
+            const float inv = 1.f / Ls;
+            *reinterpret_cast<t4 *>(static_cast<T *>(a.out) + row * D + d0) =
+                t4{T(o[0] * inv), T(o[1] * inv), T(o[2] * inv), T(o[3] * inv)};
+        };
+        int any_bad = 0;
+        for (int i = threadIdx.x; i < COLS * (D / 4); i += 64 * NW) {
+            const int c = i / (D / 4), d0 = 4 * (i % (D / 4));
+            if (col0 + c >= cols) break;
+            if (AGAIN && !bad[c]) continue;
+            const int w0 = c / (CT * 16), cl = c % (CT * 16);
+            float M = -INFINITY;
+#pragma unroll
+            for (int k = 0; k < WK; ++k) M = fmaxf(M, pml[2 * ((w0 + WC * k) * CT * 16 + cl)]);
+            float Ls = 0.f;
+            f32x4 o = {0.f, 0.f, 0.f, 0.f};
+            const float Mu = M == -INFINITY ? 0.f : M; // no key of this split seen: weights 0
+#pragma unroll
+            for (int k = 0; k < WK; ++k) {
+                const int x = (w0 + WC * k) * CT * 16 + cl;
+                const float w = __builtin_amdgcn_exp2f(pml[2 * x] - Mu);
+                Ls += pml[2 * x + 1] * w;
+                o += *reinterpret_cast<const f32x4 *>(po + x * OP + d0) * w;
+            }
+            const bool fine = finite(o[0]) && finite(o[1]) && finite(o[2]) && finite(o[3]) && finite(Ls);
+            if (!AGAIN && !fine) {
+                bad[c] = 1;
+                any_bad = 1;
+            }
+            put(c, d0, o, M, Ls);
         }
-    }
+        return !AGAIN && __syncthreads_or(any_bad) != 0;
+    };
+
+    run();
+    if (!finish(std::false_type())) return;
+    // (Addresses worked out from here on, not kept from before: registers.)
+    asm volatile("" : "+v"(lane), "+v"(n), "+v"(grp));
+    runAgain();
+    finish(std::true_type());
 }
 
 template <typename T, int D, int CT, int WC, int WK, int KU>

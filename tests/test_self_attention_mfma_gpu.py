@@ -69,18 +69,61 @@ def test_edges(Lq, S, nh, nkvh, d, dtype):
     check(run(q, k, v, scale), exact(q, k, v, scale), v, TYPES[dtype])
 
 
-# The wide tiles (64 and 128 columns) need thousands of columns: a few heads
-# of the result against float64.
-@pytest.mark.parametrize("Lq,S,nh,nkvh,d", [(1437, 1500, 12, 2, 128), (1500, 1500, 48, 4, 64)])
-def test_wide_tiles(Lq, S, nh, nkvh, d):
-    q, k, v = inputs(Lq, S, nh, nkvh, d, torch.bfloat16)
+def exact_head(q, k, v, h, scale):
+    """Head h of every query, in float64."""
+    Lq, S, kh = q.shape[0], k.shape[0], h // (q.shape[1] // k.shape[1])
+    see = torch.arange(S, device="cuda")[None] <= torch.arange(Lq, device="cuda")[:, None] + S - Lq
+    w = (q[:, h].double() @ k[:, kh].double().t().contiguous() * scale).masked_fill(~see, -math.inf)
+    return torch.softmax(w, -1) @ v[:, kh].double().contiguous()
+
+
+# The wide tiles need thousands of columns: 8622 take tiles of 64, 18000 of
+# 128 (both with a remainder). A few heads of the result against float64.
+WIDE = [(1437, 1500, 12, 2), (1500, 1501, 48, 4), (3000, 3131, 12, 2)]
+
+
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("dtype", ["f16", "bf16"])
+@pytest.mark.parametrize("Lq,S,nh,nkvh", WIDE)
+def test_wide_tiles(Lq, S, nh, nkvh, d, dtype):
+    q, k, v = inputs(Lq, S, nh, nkvh, d, TYPES[dtype])
     scale = 1 / math.sqrt(d)
     got = run(q, k, v, scale)
-    see = torch.arange(S, device="cuda")[None] <= torch.arange(Lq, device="cuda")[:, None] + S - Lq
     for h in (0, nh // 2, nh - 1):
-        kh = h // (nh // nkvh)
-        w = (q[:, h].double() @ k[:, kh].double().t().contiguous() * scale).masked_fill(~see, -math.inf)
-        check(got[:, h], torch.softmax(w, -1) @ v[:, kh].double().contiguous(), v, torch.bfloat16)
+        check(got[:, h], exact_head(q, k, v, h, scale), v, TYPES[dtype])
+
+
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("dtype", ["f16", "bf16"])
+@pytest.mark.parametrize("Lq,S,nh,nkvh", WIDE[:2])
+def test_wide_tiles_non_finite(Lq, S, nh, nkvh, d, dtype):
+    q, k, v = inputs(Lq, S, nh, nkvh, d, TYPES[dtype])
+    kb, vb = k.clone(), v.clone()
+    kb[-2:], vb[-2:] = math.nan, math.nan  # only the last two queries see these
+    vb[700, :, 9] = math.inf               # and only queries from there on this one
+    got = run(q, kb, vb, 0.1)
+    sees = torch.arange(Lq - 2, device="cuda") + S - Lq >= 700
+    for h in (0, nh - 1):
+        want = exact_head(q, k, v, h, 0.1)[:-2]
+        assert torch.isnan(got[-2:, h]).all()
+        assert (got[:-2, h, 9][sees] == math.inf).all()
+        want[:, 9] = torch.where(sees, 0.0, want[:, 9])
+        mine = got[:-2, h].clone()
+        mine[:, 9] = torch.where(sees, torch.zeros_like(mine[:, 9]), mine[:, 9])
+        check(mine, want, v, TYPES[dtype])
+
+
+# Values of 2^118, whose sums with the lazy max's weights (up to
+# 2^8) would leave f32's range: their average does not.
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+@pytest.mark.parametrize("Lq,S", [(1, 300), (350, 350), (1437, 1500)])
+def test_huge_finite_values(Lq, S, dtype):
+    q, k, v = inputs(Lq, S, 12, 2, 128, TYPES[dtype])
+    k = k * torch.linspace(0.5, 3, S, device="cuda", dtype=k.dtype)[:, None, None]
+    v = (1.0 + 0.01 * v.float().clamp(-3, 3)).mul(2.0**118).to(TYPES[dtype])
+    got = run(q, k, v, 0.1)
+    for h in (0, 7):
+        check(got[:, h].float() / 2.0**118, exact_head(q, k, v, h, 0.1) / 2.0**118, v.float() / 2.0**118, TYPES[dtype])
 
 
 # f32 sums are cut into short chains: 2-norm of the error at most 5 roundings
@@ -91,10 +134,7 @@ def test_f32_error(Lq, S, d):
     q, k, v = inputs(Lq, S, 12, 2, d, torch.float32)
     scale = 1 / math.sqrt(d)
     got = run(q, k, v, scale)
-    see = torch.arange(S, device="cuda")[None] <= torch.arange(Lq, device="cuda")[:, None] + S - Lq
-    want = torch.stack([torch.softmax((q[:, h].double() @ k[:, h // 6].double().t().contiguous() * scale)
-                                      .masked_fill(~see, -math.inf), -1) @ v[:, h // 6].double().contiguous()
-                        for h in range(12)], 1)
+    want = torch.stack([exact_head(q, k, v, h, scale) for h in range(12)], 1)
     assert float((got.double() - want).norm() / want.norm()) < 5 * 2.0**-24
 
 
