@@ -106,10 +106,17 @@ struct Acc {
     }
 };
 
-// P of one page pair for one lane's column, as bf16 (hi, and lo when SPLIT_P).
-struct PairP {
-    bf16x8 hi, lo;
+// P of one page pair for one lane's column, as PARTS bf16 parts, each what the
+// ones before it leave of the weight: to 2^-9, 2^-17 or 2^-25 of its size.
+template <int PARTS> struct PairP {
+    bf16x8 part[PARTS];
 };
+// Parts of the decode kernels' weights: one would show beside a bf16 result's
+// own rounding, two beside a 32-bit result's (2-norm of the error, 700 tokens:
+// 2.3e-3 -> 1.66e-3 and 2.3e-6 -> 2.5e-7 with the second and third part; 9.0 ->
+// 10.0 and 9.8 -> 10.9 us, and nothing where HBM is the bound: 64 x 512-8192
+// 52.1 -> 52.3).
+template <bool OUT_F32> constexpr int decodeParts() { return OUT_F32 ? 3 : 2; }
 
 // Raw scores of one page pair (K pages a, b) against the lane's column of
 // each of NT query tiles, with keys a column may not see set to -inf.
@@ -160,8 +167,9 @@ __device__ __forceinline__ void pairScoresN(float (&sv)[NT][8], const u32x4 (&ka
 // max in log2 units, sum, rescaled O) and return each pair's P. Scores enter
 // as exp2(s * scale_log2 - m): the max is taken on raw scores (the scale is
 // positive) and the scaling folds into one fma per key.
-template <bool SPLIT_P, int NP>
-__device__ __forceinline__ void softmaxUpdate(Acc &acc, const float (&sv)[NP][8], PairP (&P)[NP], float scale_log2) {
+template <int PARTS, int NP>
+__device__ __forceinline__ void softmaxUpdate(Acc &acc, const float (&sv)[NP][8], PairP<PARTS> (&P)[NP],
+                                              float scale_log2) {
     float mloc = sv[0][0];
 #pragma unroll
     for (int j = 0; j < NP; ++j)
@@ -189,23 +197,27 @@ __device__ __forceinline__ void softmaxUpdate(Acc &acc, const float (&sv)[NP][8]
         for (int i = 0; i < 8; ++i) {
             const float p = exp2Fast(__builtin_fmaf(sv[j][i], scale_log2, -m_use));
             psum += p;
-            const __bf16 hi = (__bf16)p;
-            P[j].hi[i] = hi;
-            if constexpr (SPLIT_P) P[j].lo[i] = (__bf16)(p - (float)hi);
+            float rest = p;
+#pragma unroll
+            for (int k = 0; k < PARTS; ++k) {
+                const __bf16 h = (__bf16)rest;
+                P[j].part[k][i] = h;
+                rest -= (float)h;
+            }
         }
     acc.l += psum;
 }
 
 // Scores, online softmax update and P of one page pair (see pairScores).
-template <bool SPLIT_P>
-__device__ __forceinline__ PairP scorePair(Acc &acc, const u32x4 (&ka)[4], const u32x4 (&kb)[4], const u32x4 (&qop)[4],
+template <int PARTS>
+__device__ __forceinline__ PairP<PARTS> scorePair(Acc &acc, const u32x4 (&ka)[4], const u32x4 (&kb)[4], const u32x4 (&qop)[4],
                                           int first_key, int pos, bool hasB, int grp, float scale_log2) {
     float sv[1][8];
     const u32x4(&q1)[1][4] = *reinterpret_cast<const u32x4(*)[1][4]>(&qop);
     const int p1[1] = {pos};
     pairScoresN<1>(sv, ka, kb, q1, first_key, p1, hasB, grp);
-    PairP P[1];
-    softmaxUpdate<SPLIT_P, 1>(acc, sv, P, scale_log2);
+    PairP<PARTS> P[1];
+    softmaxUpdate<PARTS, 1>(acc, sv, P, scale_log2);
     return P[0];
 }
 
@@ -227,17 +239,17 @@ __device__ __forceinline__ void maskStaleV(u32x4 (&va)[4], u32x4 (&vb)[4], int f
 }
 
 // O^T += V^T . P^T for one page pair (V pages a, b already masked).
-template <bool SPLIT_P>
-__device__ __forceinline__ void accumulatePV(Acc &acc, const u32x4 (&va)[4], const u32x4 (&vb)[4], const PairP &P) {
+template <int PARTS>
+__device__ __forceinline__ void accumulatePV(Acc &acc, const u32x4 (&va)[4], const u32x4 (&vb)[4],
+                                             const PairP<PARTS> &P) {
 #pragma unroll
     for (int s = 0; s < 4; ++s) {
         const bf16x8 v0 = asBf16(u32x4{va[s][0], va[s][1], vb[s][0], vb[s][1]});
         const bf16x8 v1 = asBf16(u32x4{va[s][2], va[s][3], vb[s][2], vb[s][3]});
-        acc.o[2 * s] = mfma(v0, P.hi, acc.o[2 * s]);
-        acc.o[2 * s + 1] = mfma(v1, P.hi, acc.o[2 * s + 1]);
-        if constexpr (SPLIT_P) {
-            acc.o[2 * s] = mfma(v0, P.lo, acc.o[2 * s]);
-            acc.o[2 * s + 1] = mfma(v1, P.lo, acc.o[2 * s + 1]);
+#pragma unroll
+        for (int k = 0; k < PARTS; ++k) {
+            acc.o[2 * s] = mfma(v0, P.part[k], acc.o[2 * s]);
+            acc.o[2 * s + 1] = mfma(v1, P.part[k], acc.o[2 * s + 1]);
         }
     }
 }
@@ -261,29 +273,28 @@ __device__ __forceinline__ void maskStaleVPacked(u32x4 (&v0)[4], u32x4 (&v1)[4],
     }
 }
 
-template <bool SPLIT_P>
+template <int PARTS>
 __device__ __forceinline__ void accumulatePVPacked(Acc &acc, const u32x4 (&v0)[4], const u32x4 (&v1)[4],
-                                                   const PairP &P) {
+                                                   const PairP<PARTS> &P) {
 #pragma unroll
     for (int s = 0; s < 4; ++s) {
-        acc.o[2 * s] = mfma(asBf16(v0[s]), P.hi, acc.o[2 * s]);
-        acc.o[2 * s + 1] = mfma(asBf16(v1[s]), P.hi, acc.o[2 * s + 1]);
-        if constexpr (SPLIT_P) {
-            acc.o[2 * s] = mfma(asBf16(v0[s]), P.lo, acc.o[2 * s]);
-            acc.o[2 * s + 1] = mfma(asBf16(v1[s]), P.lo, acc.o[2 * s + 1]);
+#pragma unroll
+        for (int k = 0; k < PARTS; ++k) {
+            acc.o[2 * s] = mfma(asBf16(v0[s]), P.part[k], acc.o[2 * s]);
+            acc.o[2 * s + 1] = mfma(asBf16(v1[s]), P.part[k], acc.o[2 * s + 1]);
         }
     }
 }
 
 // Consume one page pair: scores, online softmax and P.V (see scorePair for
 // the arguments; ctx = keys in cache, whose later slots get zeroed V).
-// SPLIT_P: P enters P.V as hi + lo bf16 parts (fp32-accurate) or as one bf16.
-template <bool SPLIT_P>
+// PARTS: the bf16 parts as which P enters P.V.
+template <int PARTS>
 __device__ __forceinline__ void consumePair(Acc &acc, PagePair &r, const u32x4 (&qop)[4], int first_key, int pos,
                                            int ctx, bool hasB, int grp, float scale_log2) {
-    const PairP P = scorePair<SPLIT_P>(acc, r.ka, r.kb, qop, first_key, pos, hasB, grp, scale_log2);
+    const PairP<PARTS> P = scorePair<PARTS>(acc, r.ka, r.kb, qop, first_key, pos, hasB, grp, scale_log2);
     maskStaleV(r.va, r.vb, first_key, ctx, hasB, grp);
-    accumulatePV<SPLIT_P>(acc, r.va, r.vb, P);
+    accumulatePV<PARTS>(acc, r.va, r.vb, P);
 }
 
 // Output dims of lane (n, grp) for block i: 16*i + 4*grp + {0..3}.

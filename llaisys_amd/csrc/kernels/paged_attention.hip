@@ -49,6 +49,9 @@ constexpr int kWaves = 8;                                    // waves (groups) p
 constexpr int kStagePairs = 2;                               // page pairs per LDS stage (one barrier each)
 constexpr int kRecordFloats = kTiles * 16 * (kHeadDim + 2); // O for the group's columns, then (m, l)
 
+// bf16 parts of the prompt tiles' weights.
+template <bool OUT_F32> constexpr int weightParts() { return OUT_F32 ? 2 : 1; }
+
 constexpr int kQueueSplitWord = kPrefillQueueWords - 1; // a cache line past the counters
 
 struct Args {
@@ -318,9 +321,9 @@ __device__ __forceinline__ void prefillItem(const Args &a, StageBuf &kvs, int b,
 #pragma unroll
                         for (int e = 0; e < 8; ++e) sv[k][j][e] = svj[k][e];
                 }
-                PairP P[kTiles][kSoft];
+                PairP<weightParts<OUT_F32>()> P[kTiles][kSoft];
 #pragma unroll
-                for (int k = 0; k < kTiles; ++k) softmaxUpdate<OUT_F32, kSoft>(acc[k], sv[k], P[k], a.scale_log2);
+                for (int k = 0; k < kTiles; ++k) softmaxUpdate<weightParts<OUT_F32>(), kSoft>(acc[k], sv[k], P[k], a.scale_log2);
 #pragma unroll
                 for (int j = 0; j < kSoft; ++j) {
                     const int pp = ps + 2 * (sg + j);
@@ -335,7 +338,7 @@ __device__ __forceinline__ void prefillItem(const Args &a, StageBuf &kvs, int b,
                     }
                     maskStaleVPacked(v0, v1, pp * 16, t.ctx, hasB, grp);
 #pragma unroll
-                    for (int k = 0; k < kTiles; ++k) accumulatePVPacked<OUT_F32>(acc[k], v0, v1, P[k][j]);
+                    for (int k = 0; k < kTiles; ++k) accumulatePVPacked<weightParts<OUT_F32>()>(acc[k], v0, v1, P[k][j]);
                 }
             }
         }
@@ -447,7 +450,7 @@ __device__ __forceinline__ void decodeItem(const Args &a, StageBuf &kvs, int b, 
                     const int k = k0 + st;
                     if (k < cnt) {
                         const int j = base + k;
-                        consumePair<OUT_F32>(acc, ring[st], qop, 32 * j, c - 1, c, 2 * j + 1 < np, grp, a.scale_log2);
+                        consumePair<decodeParts<OUT_F32>()>(acc, ring[st], qop, 32 * j, c - 1, c, 2 * j + 1 < np, grp, a.scale_log2);
                     }
                     issue(st, k + 2);
                 }

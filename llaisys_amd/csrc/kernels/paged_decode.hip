@@ -347,7 +347,7 @@ __global__ void __launch_bounds__(64)
                 u32x4 qop[4];
 #pragma unroll
                 for (int t = 0; t < 4; ++t) qop[t] = n < G ? ring.q[st][t] : u32x4{0, 0, 0, 0};
-                consumePair<OUT_F32>(acc, ring.pp[st], qop, 32 * j, c - 1, c, hasB, grp, a.scale_log2);
+                consumePair<decodeParts<OUT_F32>()>(acc, ring.pp[st], qop, 32 * j, c - 1, c, hasB, grp, a.scale_log2);
             }
             issue(st, k + NSTAGE);
         }
@@ -776,7 +776,7 @@ __global__ void __launch_bounds__(64 * kUnitWaves)
                 const int k = k0 + st;
                 if (k < cnt_c) {
                     const int j = wave + kUnitWaves * (base + k);
-                    consumePair<OUT_F32>(acc, ring[st], qop, 32 * j, c - 1, c, 2 * j + 1 < np, grp, a.scale_log2);
+                    consumePair<decodeParts<OUT_F32>()>(acc, ring[st], qop, 32 * j, c - 1, c, 2 * j + 1 < np, grp, a.scale_log2);
                 }
                 issue(st, k + NSTAGE);
             }
@@ -805,7 +805,7 @@ __global__ void __launch_bounds__(64 * kUnitWaves)
             __builtin_amdgcn_wave_barrier();
             const int j = npr - 1;
             patchNewToken(ring[0], kflat, vflat, tok, 2 * j == np - 1, lane);
-            consumePair<OUT_F32>(acc, ring[0], qop, 32 * j, c - 1, c, 2 * j + 1 < np, grp, a.scale_log2);
+            consumePair<decodeParts<OUT_F32>()>(acc, ring[0], qop, 32 * j, c - 1, c, 2 * j + 1 < np, grp, a.scale_log2);
             // Stores into the page slot for later steps: lanes 0-15 the k
             // chunks [d / 8][tok] (16 B each), every lane its 2 v dims.
             if (unsigned(blk) >= unsigned(a.num_blocks)) {

@@ -41,6 +41,24 @@ def test_one_long_sequence(tokens, fn):
     check(make_case(tokens, np.array([tokens], np.int32)), fn)
 
 
+# 2-norm of the error. bf16: the result's own rounding (1.65e-3 for values spread
+# over their exponents) and a tenth for the weights' two parts; with one part
+# 2.0e-3 to 2.4e-3. f32: sums in 32 bits (about 2^-21); with two parts 1.7e-6 and more.
+@pytest.mark.parametrize("lens", [[700], [300], [4000], [200, 450, 700], [100] * 40 + [800] * 30])
+def test_weights_do_not_show(lens):
+    case = make_case(8, np.array(lens, np.int32))
+    q = queries(5, case.B, case.nh)
+    ref = np.empty(q.shape)  # in 64 bits (the oracle's own 32-bit sums are off by 1.3e-6 at 4000 tokens)
+    for b, n in enumerate(lens):
+        k, v = (from_bits(log[case.table[b, :(n + 15) // 16]].swapaxes(1, 2).reshape(-1, case.nkvh, 128)[:n]).double().cpu()
+                for log in (case.k_log, case.v_log))
+        for h in range(case.nh):
+            w = torch.softmax(k[:, h // 6] @ from_bits(q[b, h]).double().cpu() * SCALE, 0)
+            ref[b, h] = (w @ v[:, h // 6]).numpy()
+    for dtype, most in ((torch.bfloat16, 1.8e-3), (torch.float32, 2.0**-20)):
+        assert np.linalg.norm(run(case, q, dtype) - ref) < most * np.linalg.norm(ref), dtype
+
+
 def test_a_long_sequence_among_short_ones():
     check(make_case(3, np.array([3, 900, 17, 20000, 33, 1, 64, 2500], np.int32)))
 
