@@ -405,11 +405,46 @@ __global__ void __launch_bounds__(64 * WGM * WGN) gemmKernel(GemmParams p) {
             }
             __builtin_amdgcn_sched_group_barrier(0x008, kMfmas - kPer * kReads > 0 ? kMfmas - kPer * kReads : 0, 0);
         };
+        // f32: an MFMA adds its four products to one running sum, so the error
+        // goes with the root of the k loop's length. The sums start afresh
+        // every 16 k tiles (256 k), but where K is split in 8, which is short
+        // enough: 400 x 1536 x 8960 9.8e-7 -> 3.0e-7 of the result's 2-norm,
+        // 1024 x 1536 x 1536 7.0e-7 -> 2.9e-7, for 1 to 3 % of the time. (Two
+        // nested loops took 5 to 9 %.)
+        constexpr int kFresh = T == ElemType::F32 ? TN : 1;
+        f32x4 total[kFresh][TM];
+        const bool fresh = T == ElemType::F32 && p.splits < 8;
+#pragma unroll
+        for (int i = 0; i < kFresh; ++i)
+#pragma unroll
+            for (int j = 0; j < TM; ++j) total[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
         u32x4 a0[TN], b0[TM], a1[TN], b1[TM];
         readFrags(0, a0, b0);
+        // The next fresh start: past the end for none.
+        int next = fresh ? 16 : 0x7fffffff;
         for (int kt = 0; kt < nk; kt += 2) {
+            if constexpr (T == ElemType::F32) {
+                if (kt == next) {
+                    next += 16;
+#pragma unroll
+                    for (int i = 0; i < TN; ++i)
+#pragma unroll
+                        for (int j = 0; j < TM; ++j) {
+                            total[i][j] += acc[i][j];
+                            acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+                        }
+                }
+            }
             step(kt, a0, b0, a1, b1);
             if (kt + 1 < nk) step(kt + 1, a1, b1, a0, b0);
+        }
+        if constexpr (T == ElemType::F32) {
+            if (fresh) {
+#pragma unroll
+                for (int i = 0; i < TN; ++i)
+#pragma unroll
+                    for (int j = 0; j < TM; ++j) acc[i][j] += total[i][j];
+            }
         }
     } else {
         for (int kt = 0; kt < nk; ++kt) {
@@ -674,16 +709,22 @@ __global__ void __launch_bounds__(64 * NW) gemmFewRowsKernel(GemmParams p) {
                     f.x[u][t][j] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(xr, int(in ? xbase[t] + k : kMasked), 0, 0));
             }
     };
-    f32x4 acc[MT];
+    // f32: a sum per segment of a set, so that the chains of additions stay
+    // short (16 x 2048 x 1536: error 3.6e-7 -> 1.9e-7 of the result's 2-norm).
+    constexpr int SUMS = T == ElemType::F32 ? U : 1;
+    f32x4 acc[SUMS][MT];
 #pragma unroll
-    for (int t = 0; t < MT; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int u = 0; u < SUMS; ++u)
+#pragma unroll
+        for (int t = 0; t < MT; ++t) acc[u][t] = f32x4{0.f, 0.f, 0.f, 0.f};
     auto use = [&](const Set &f) {
 #pragma unroll
         for (int u = 0; u < U; ++u)
 #pragma unroll
             for (int j = 0; j < 2; ++j)
 #pragma unroll
-                for (int t = 0; t < MT; ++t) acc[t] = mfmaPiece<T>(f.w[u][j], f.x[u][t][j], acc[t]);
+                for (int t = 0; t < MT; ++t)
+                    acc[u % SUMS][t] = mfmaPiece<T>(f.w[u][j], f.x[u][t][j], acc[u % SUMS][t]);
     };
     Set a, b;
     load(a, 0);
@@ -694,11 +735,15 @@ __global__ void __launch_bounds__(64 * NW) gemmFewRowsKernel(GemmParams p) {
         if (s + 2 * U < steps) load(a, s + 2 * U);
         use(b);
     }
+#pragma unroll
+    for (int u = 1; u < SUMS; ++u)
+#pragma unroll
+        for (int t = 0; t < MT; ++t) acc[0][t] += acc[u][t];
     // Lane: rows 4 grp + i of the tile, column n; in quadrant (a, a) both belong to group a.
     if ((4 * grp) / R == n / R) {
 #pragma unroll
         for (int t = 0; t < MT; ++t)
-            *reinterpret_cast<f32x4 *>(&part[wave * KR + n / R][t * R + n % R][(4 * grp) % R]) = acc[t];
+            *reinterpret_cast<f32x4 *>(&part[wave * KR + n / R][t * R + n % R][(4 * grp) % R]) = acc[0][t];
     }
     __syncthreads();
     for (int i = threadIdx.x; i < MT * R * R; i += 64 * NW) {
