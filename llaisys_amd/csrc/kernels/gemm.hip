@@ -960,13 +960,22 @@ bool w8() {
 //   M = 5          5.9 / 10.4  16.0 / 32.9                17.4 / 28.4
 //   M = 16         8.5 / 10.8  19.0 / 33.4                34.3 / 28.7
 // Every workgroup reads the rows of X for its few rows of W, so with M the
-// lead goes to the tiles, first where W is large.
+// lead goes to the tiles, first where W is large. And a workgroup walks all of
+// K, which the tiles split: past some K the tiles lead however narrow W is
+// (512 columns: M = 32 K = 2048 7.3 / 7.6, 3072 9.9 / 7.9, 8192 22.9 / 10.2; M =
+// 16 K = 3072 7.0 / 7.7, 4096 8.8 / 8.2, 8192 15.8 / 10.0; M = 8 K = 8192 8.9 /
+// 9.7, 256 columns 16384 16.0 / 13.3). Wide W of short rows makes
+// workgroups that have next to nothing to do (8960 columns, K = 128, f32, M = 4
+// 9.6 / 4.9; K = 512, 16-bit, M = 2 5.0 / 4.7, M = 4 5.5 / 4.8).
 bool takesFewRows(ElemType t, const GemmParams &p) {
     const long nk = long(p.N) * p.K;
     if ((reinterpret_cast<uintptr_t>(p.x) | reinterpret_cast<uintptr_t>(p.w)) % 16 || p.swiglu) return false;
-    if (p.M <= 4) return true;
-    if (t == ElemType::F32) return p.M <= 8 || (p.M <= 16 && p.K <= 4096);
-    return (p.M <= 8 && p.N <= 4096) || (p.M <= 32 && nk <= (1L << 22));
+    if (t == ElemType::F32) return p.M <= 8 ? p.N <= 2048 || p.K >= 512 : p.M <= 16 && p.K <= 3072;
+    if (p.M <= 2) return p.N <= 4096 || p.K >= 1024;
+    if (p.M <= 4) return p.N <= 4096 && nk < (1L << 24);
+    if (p.M <= 8) return p.N <= 4096 && p.K <= 8192 && nk < (1L << 24);
+    if (p.M <= 16) return p.K <= 3072 && nk <= (1L << 22);
+    return p.M <= 32 && p.K <= 2048 && nk <= (1L << 22);
 }
 
 template <ElemType T, int R, int NW, int MT> void launchFewRowsAs(const GemmParams &p, hipStream_t s) {

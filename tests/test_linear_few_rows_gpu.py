@@ -40,12 +40,15 @@ def test_rows_and_widths(M, N, K, dtype):
 # both sides of the dispatch's lines, and a long K
 @pytest.mark.parametrize("dtype", list(TYPES))
 @pytest.mark.parametrize("M,N,K", [(1, 4099, 8960), (3, 64, 16384), (8, 4096, 1024), (8, 4097, 1024), (16, 2048, 2048),
-                                   (16, 2056, 2048), (16, 128, 4096), (16, 128, 4104), (32, 4096, 1024), (32, 4096, 1032)])
+                                   (16, 2056, 2048), (16, 128, 4096), (16, 128, 4104), (32, 4096, 1024), (32, 4096, 1032),
+                                   (2, 4104, 1016), (2, 4104, 1024), (4, 4096, 4088), (4, 4096, 4096), (4, 2056, 504),
+                                   (4, 2056, 512), (8, 70, 8192), (8, 70, 8200), (16, 70, 3072), (16, 70, 3080),
+                                   (32, 70, 2048), (32, 70, 2056)])
 def test_around_the_dispatch(M, N, K, dtype):
     check(M, N, K, dtype)
 
 
-def test_no_products():
+def test_a_single_piece_of_k():
     check(3, 5, 8, "f32", bias=False)
 
 
