@@ -860,6 +860,11 @@ constexpr int kMinSplitTiles = 8;            // k tiles (of 64 B) per split at l
 constexpr int kMaxSplits = 8;
 constexpr double kReduceBytesPerUs = 5.0e6;
 constexpr double kReduceLaunchUs = 2.5;
+// What a finer split of the same 16-bit tile has to promise: of two within that
+// of each other the coarser was the faster (us: 64 x 1536 x 1536 in 4 / 5 parts
+// 7.4 / 7.9), above all where the finer one puts two workgroups on a CU (9 x 4096
+// x 8192 in 4 / 8 14.2 / 15.2, 9 x 4096 x 6144 12.1 / 13.3).
+constexpr double kFinerGain = 0.98, kShareGain = 0.95;
 
 double roundsUs(ElemType t, int tile, long workgroups, long cus, double k) {
     const TileShape &c = kTiles[tile];
@@ -892,7 +897,9 @@ Plan planGemm(ElemType t, int M, int N, int K, bool no_split = false, bool swigl
             double tm = roundsUs(t, i, mt * nt * sp, cus, double(K) / sp);
             if (sp > 1)
                 tm += kReduceLaunchUs + (2.0 * sp * 4.0 + es) * double(M) * N / kReduceBytesPerUs;
-            if (tm < best_t) {
+            const bool finer = t != ElemType::F32 && best.tile == i && best.splits > 1 && sp > best.splits;
+            const double gain = !finer ? 1.0 : i == kTile64 && mt * nt * sp > cus ? kShareGain : kFinerGain;
+            if (tm < gain * best_t) {
                 best_t = tm;
                 best.tile = i;
                 best.mtiles = int(mt);
