@@ -15,7 +15,7 @@
 // A workgroup of 4 or 8 waves (2 x 2, 2 x 4 or 4 x 2) owns a BM x BN tile
 // of Y; each wave one sub-tile of it (64 x 48 to 128 x 64). K advances in
 // tiles of 128 B per row (64 16-bit elements; f32: 64 B, 16 elements)
-// through an LDS ring of two stages (f32: four): each wave moves whole 1 KiB
+// through an LDS ring of two to four stages (f32: four): each wave moves whole 1 KiB
 // blocks of X and W rows straight from global memory into LDS by 16 B
 // global_load_lds (buffer loads: out-of-range rows and k come back as zeros,
 // so edge tiles need no other guard), and one barrier per stage both
@@ -799,7 +799,7 @@ bool pipelined() {
     return v;
 }
 
-// 16-bit tiles move k in 128 B row pieces (two stages) unless
+// 16-bit tiles move k in 128 B row pieces (two to four stages, wideStages) unless
 // LLAISYS_GEMM_WIDE_K=0 (64 B pieces, four stages).
 bool wideK() {
     static const bool v = [] { const char *e = std::getenv("LLAISYS_GEMM_WIDE_K"); return !(e && e[0] == '0'); }();
@@ -916,8 +916,10 @@ Plan planGemm(ElemType t, int M, int N, int K, bool no_split = false, bool swigl
 // 560 tiles of 256 x 256 in three rounds on 256 CUs, the last under a fifth
 // full) runs as two launches instead: columns [0, na) on the plan's tiles in
 // whole rounds, the rest on their own (smaller) tiles, when the model prices
-// the two below the one. Splits of K are left alone. na is a multiple of the
-// tile width (so of 64: whole SwiGLU pairs, 16 B aligned rows).
+// the two below the one. Splits of K are left alone. A round is what roundsUs
+// counts as one: two workgroups a CU for 16-bit 64 x 64 tiles. na is a multiple
+// of the tile width: 16 B aligned rows, and whole SwiGLU pairs, since the fused
+// gate-up takes no narrow tiles.
 constexpr double kSecondLaunchUs = 3.0;
 struct ColumnSplit {
     int na = 0; // 0: one launch
@@ -928,9 +930,10 @@ ColumnSplit splitColumns(ElemType t, int M, int N, int K, const Plan &one, bool 
     static const bool on = [] { const char *e = std::getenv("LLAISYS_GEMM_COLUMN_SPLIT"); return !(e && e[0] == '0'); }();
     if (!on || one.splits != 1 || N % 8 != 0) return cs; // (vector stores need rows of whole 16 B)
     const long cus = cusOf();
-    const long tiles = long(one.mtiles) * one.ntiles, rounds = (tiles + cus - 1) / cus;
-    if (rounds < 2 || tiles % cus == 0) return cs;
-    const int nta = int((rounds - 1) * cus / one.mtiles); // column tiles that fill rounds - 1 rounds
+    const long full = one.tile == kTile64 && t != ElemType::F32 ? 2 * cus : cus; // workgroups of a round
+    const long tiles = long(one.mtiles) * one.ntiles, rounds = (tiles + full - 1) / full;
+    if (rounds < 2 || tiles % full == 0) return cs;
+    const int nta = int((rounds - 1) * full / one.mtiles); // column tiles that fill rounds - 1 rounds
     if (nta <= 0 || nta >= one.ntiles) return cs;
     const int na = nta * kTiles[one.tile].bn;
     const Plan a = planGemm(t, M, na, K, true, swiglu), b = planGemm(t, M, N - na, K, true, swiglu);
