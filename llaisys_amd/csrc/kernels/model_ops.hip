@@ -186,11 +186,16 @@ __global__ void __launch_bounds__(kThreads) rmsNormRowKernel(T *out, const T *x,
 
 // Rotate halves: for j < d/2, phi = pos / theta^(2j/d) computed in fp32 as the
 // reference formula does; a' = a cos - b sin, b' = b cos + a sin.
-// The block's token has one angle per j, whatever the head: they are worked
-// out once (powf, a division and sincosf each) and shared through LDS. VEC:
-// 16 B pieces, where half a head is whole pieces and the tensors are aligned.
-// 4096 tokens x 12 heads of 128 bf16: 19.7 -> 6.6 us.
-constexpr int kRopeHalf = 512; // angles kept in LDS; larger heads work theirs out in place
+// The block's token has one angle per j, whatever the head. kShared: they are
+// worked out once (powf, a division and sincosf each) and shared through LDS;
+// kPieces: and the rows move in 16 B pieces, where half a head is whole pieces
+// and the tensors are aligned. 4096 tokens x 12 heads of 128 bf16: 19.7 -> 6.6
+// us. kOwn: every element works its own out, the shorter way where no more than
+// one wave has something to do or one head shares with none (us, kOwn / kPieces:
+// 5000 tokens x 2 heads of 16 3.9 / 5.1, 3000 x 1 of 256 4.4 / 4.7; 4096 x 2 of
+// 128 5.3 / 4.7), and for heads too large for the LDS.
+constexpr int kRopeHalf = 512; // angles kept in LDS
+enum RopeMode { kOwn, kShared, kPieces };
 
 __device__ __forceinline__ float2 ropeAngle(float p, int j, int d, float theta) {
     float s, c;
@@ -198,14 +203,14 @@ __device__ __forceinline__ float2 ropeAngle(float p, int j, int d, float theta) 
     return make_float2(s, c);
 }
 
-template <typename T, bool VEC>
+template <typename T, RopeMode MODE>
 __global__ void __launch_bounds__(kThreads) ropeKernel(T *out, const T *in, const int64_t *pos, int nhead, int d, float theta) {
-    __shared__ float2 trig[kRopeHalf];
+    __shared__ float2 trig[MODE == kOwn ? 1 : kRopeHalf];
+    constexpr bool VEC = MODE == kPieces;
     const size_t tok = blockIdx.x;
     const int half = d / 2;
     const float p = float(pos[tok]);
-    const bool shared = half <= kRopeHalf;
-    if (shared) {
+    if constexpr (MODE != kOwn) {
         for (int j = threadIdx.x; j < half; j += kThreads) trig[j] = ropeAngle(p, j, d, theta);
         __syncthreads();
     }
@@ -227,7 +232,7 @@ __global__ void __launch_bounds__(kThreads) ropeKernel(T *out, const T *in, cons
             ra.store(out + base);
             rb.store(out + base + half);
         } else {
-            const float2 sc = shared ? trig[j] : ropeAngle(p, j, d, theta);
+            const float2 sc = MODE == kShared ? trig[j] : ropeAngle(p, j, d, theta);
             const float a = ld(in, base), b = ld(in, base + half);
             st(out, base, a * sc.y - b * sc.x);
             st(out, base + half, b * sc.y + a * sc.x);
@@ -402,10 +407,13 @@ template <typename T> struct RmsL {
 template <typename T> struct RopeL {
     static void run(void *o, const void *x, const int64_t *pos, size_t ntok, int nhead, int d, float theta, hipStream_t s) {
         if (!ntok) return;
-        if ((d / 2) % Vec<T>::N == 0 && d / 2 <= kRopeHalf && aligned16({o, x}))
-            hipLaunchKernelGGL((ropeKernel<T, true>), dim3(ntok), dim3(kThreads), 0, s, (T *)o, (const T *)x, pos, nhead, d, theta);
+        const int half = d / 2;
+        if (half > kRopeHalf || nhead == 1 || nhead * half <= 64)
+            hipLaunchKernelGGL((ropeKernel<T, kOwn>), dim3(ntok), dim3(kThreads), 0, s, (T *)o, (const T *)x, pos, nhead, d, theta);
+        else if (half % Vec<T>::N == 0 && aligned16({o, x}))
+            hipLaunchKernelGGL((ropeKernel<T, kPieces>), dim3(ntok), dim3(kThreads), 0, s, (T *)o, (const T *)x, pos, nhead, d, theta);
         else
-            hipLaunchKernelGGL((ropeKernel<T, false>), dim3(ntok), dim3(kThreads), 0, s, (T *)o, (const T *)x, pos, nhead, d, theta);
+            hipLaunchKernelGGL((ropeKernel<T, kShared>), dim3(ntok), dim3(kThreads), 0, s, (T *)o, (const T *)x, pos, nhead, d, theta);
     }
 };
 template <typename T> struct EmbL {
