@@ -391,9 +391,11 @@ template <typename T> struct RmsL {
         constexpr int N = Vec<T>::N;
         const bool vec = d % N == 0 && aligned16({o, x, w});
         const dim3 grid(unsigned((rows + kThreads / 64 - 1) / (kThreads / 64)));
-        // Up to four rows a CU a block per row is the shorter chain (48 rows in
-        // front of the LM head: 98.35 us against 97.8).
-        const bool many = rows > 1024;
+        // A block per row spreads few rows over more waves: 2048 x 4096 in 16 bits
+        // 5.4 us and 5.9 with a wave per row, 1025 x 4096 4.1 and 4.2; rows past
+        // four pieces a lane need more of them (2100 x 4096 6.1 / 6.8, 3000 8.7 /
+        // 8.6, 4096 11.9 / 11.0) than shorter ones (3000 x 1536 4.8 / 4.4).
+        const bool many = rows > (d <= 64 * 4 * N ? 2048 : 3072);
         if (many && vec && d <= 64 * 4 * N)
             hipLaunchKernelGGL((rmsNormRowKernel<T, 4>), grid, dim3(kThreads), 0, s, (T *)o, (const T *)x, (const T *)w, rows, d, eps);
         else if (many && vec && d <= 64 * 8 * N)
