@@ -622,7 +622,7 @@ void Qwen2Model::forward(size_t T, size_t B, bool decode_only) {
                                     int(num_blocks_), scale, rt.errorWord(), s);
             else
                 ops::pagedAttention(a3, q3, k_pool_[l], v_pool_[l], table_, ctx_after_, decode_only ? nullptr : cu_,
-                                    scale);
+                                    scale, decode_only);
         }
         if (px)
             K::packedXGemm(u16(x_), u16(ap_), u16(L.o_wp), M, hs, q, true, s, fused_mlp ? u16(xp_) : nullptr);

@@ -294,7 +294,8 @@ AttnDims checkAttention(const char *op, const tensor_t &out, const tensor_t &q, 
 } // namespace
 
 void pagedAttention(const tensor_t &out, const tensor_t &q, const tensor_t &k_pool, const tensor_t &v_pool,
-                    const tensor_t &block_table, const tensor_t &ctx_len, const tensor_t &cu_q, float scale) {
+                    const tensor_t &block_table, const tensor_t &ctx_len, const tensor_t &cu_q, float scale,
+                    bool stream_k) {
     const char *op = cu_q ? "paged_attention_varlen" : "paged_attention";
     const auto [T, nh, nkvh, B] = checkAttention(op, out, q, k_pool, v_pool, block_table, ctx_len, cu_q);
     const bool host = onHost(op, {&out, &q, &k_pool, &v_pool, &block_table, &ctx_len, &cu_q});
@@ -319,7 +320,7 @@ void pagedAttention(const tensor_t &out, const tensor_t &q, const tensor_t &k_po
     const auto *tab = reinterpret_cast<const int32_t *>(block_table->data());
     const auto *ctx = reinterpret_cast<const int32_t *>(ctx_len->data());
     const int nb = int(k_pool->shape()[0]);
-    if (!cu_q && K::unitDecodeTakes(int(B), int(nkvh), max_pages)) {
+    if (!cu_q && !stream_k && K::unitDecodeTakes(int(B), int(nkvh), max_pages)) {
         K::pagedDecodeUnits(out->data(), f32, qp, kp, vp, tab, ctx, int(B), int(nh), int(nkvh), max_pages, nb, scale,
                             rt.errorWord(), rt.stream(), nullptr, true);
         return;

@@ -19,9 +19,11 @@ void pagedKVAppendGather(const tensor_t &k_out, const tensor_t &v_out, const ten
 
 void pagedKVCopyBlocks(const tensor_t &k_pool, const tensor_t &v_pool, const tensor_t &pairs);
 
+// stream_k: decode keeps the stream-K kernel also where the block table's width
+// would choose the one workgroup per sequence and kv head.
 void pagedAttention(const tensor_t &out, const tensor_t &q, const tensor_t &k_pool, const tensor_t &v_pool,
                     const tensor_t &block_table, const tensor_t &ctx_len, const tensor_t &cu_q /* null = decode */,
-                    float scale);
+                    float scale, bool stream_k = false);
 
 // Decode attention (pagedAttention with cu_q null) with no device allocation:
 // split records in the decode kernel's fixed per-GPU scratch. AMD tensors only.

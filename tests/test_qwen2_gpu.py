@@ -180,6 +180,26 @@ def test_decode_attention_one_workgroup_per_unit(monkeypatch, shape, units, rope
     assert np.array_equal(np.asarray(multi), np.asarray(single, np.int64))
 
 
+def test_decode_units_switch_reaches_the_other_kernel(monkeypatch):
+    # With the epilogue in a launch of its own, LLAISYS_DECODE_UNITS is what
+    # chooses the decode attention, also in block tables narrow enough for the
+    # op to choose by itself: one workgroup per unit sums each unit's pages in
+    # another order than the stream-K kernel does, which shows in some logits.
+    monkeypatch.setenv("LLAISYS_DECODE_UNIT_ROPE", "0")
+    outs = []
+    for units in ("1", "0"):
+        monkeypatch.setenv("LLAISYS_DECODE_UNITS", units)
+        model, _ = build("tiny", num_blocks=70 * 40 + 8)
+        ids = [model.create_sequence()[0] for _ in range(70)]
+        prompts = [prompt(300 + (i * 37) % 291, model.meta.voc, 500 + i) for i in range(70)]
+        for s in range(0, 70, 10):
+            model.step(ids[s:s + 10], prompts[s:s + 10])
+        model.step(ids, [[7]] * 70)
+        outs.append(to_torch(model.logits()).float().clone())
+    assert not torch.equal(outs[0], outs[1])
+    assert float((outs[0] - outs[1]).norm() / outs[0].norm()) < 1e-2
+
+
 def test_fused_qkv_epilogue_matches_separate_launch(monkeypatch):
     # The unit attention with the QKV epilogue fused in against the same
     # model with qkvRopeAppend in its own launch, step by step over 4 decode
