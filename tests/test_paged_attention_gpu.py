@@ -46,10 +46,12 @@ def check(got_f32, got_bf16, ref):
     assert abs_err <= BF16_ABS, f"bf16 abs error {abs_err:.3g}"
 
 
+# 17 pages take the one workgroup per unit, 77 the stream-K kernel.
+@pytest.mark.parametrize("extra_pages", [0, 60])
 @pytest.mark.parametrize("nh,nkvh", [(12, 2), (16, 1), (4, 4), (8, 2)])
-def test_decode_edge_lengths(nh, nkvh):
+def test_decode_edge_lengths(nh, nkvh, extra_pages):
     ctx = np.array([1, 2, 15, 16, 17, 31, 32, 33, 63, 64, 65, 100, 257], np.int32)
-    case = make_case(10 + nh, ctx, nh=nh, nkvh=nkvh)
+    case = make_case(10 + nh, ctx, nh=nh, nkvh=nkvh, extra_pages=extra_pages)
     q = queries(99, case.B, nh)
     ref = oracle.paged_attention(q, case.k_log, case.v_log, case.table, case.ctx, SCALE)
     check(run_decode(case, q, torch.float32), run_decode(case, q, torch.bfloat16), ref)
@@ -77,7 +79,9 @@ def test_decode_record_slots_reset_between_calls(monkeypatch):
     a = make_case(51, oracle.randint(14, 64, 512, 8192).astype(np.int32))
     qa = queries(52, a.B, 12)
     ref_a = oracle.paged_attention(qa, a.k_log, a.v_log, a.table, a.ctx, SCALE, nthreads=16)
-    b = make_case(53, np.array([30000, 40], np.int32))  # one unit spread over many waves: overflow
+    # 2188 page pairs a unit, 64 at most to a wave: more pieces than the 32
+    # slots of a small batch, so these units overflow to the per-wave records
+    b = make_case(53, np.array([70000, 40], np.int32))
     qb = queries(54, b.B, 12)
     ref_b = oracle.paged_attention(qb, b.k_log, b.v_log, b.table, b.ctx, SCALE)
     c = make_case(55, oracle.randint(15, 9, 1, 3000).astype(np.int32))
@@ -86,12 +90,21 @@ def test_decode_record_slots_reset_between_calls(monkeypatch):
     # a small batch whose units use the slots (one pair per wave), so its
     # records land where a larger batch's slot headers would sit in a shared
     # layout
-    d = make_case(57, np.array([100, 150, 200, 250], np.int32))
+    # (the table is wide enough for the stream-K kernel)
+    d = make_case(57, np.array([100, 150, 200, 250], np.int32), extra_pages=60)
     qd = queries(58, d.B, 12)
     ref_d = oracle.paged_attention(qd, d.k_log, d.v_log, d.table, d.ctx, SCALE)
+    # past 512 units a unit has 8 slots instead of 32, so the headers lie
+    # elsewhere; one sequence is cut finer than that
+    ctx_e = oracle.randint(18, 270, 1, 200).astype(np.int32)
+    ctx_e[100] = 9000
+    e = make_case(59, ctx_e)
+    qe = queries(60, e.B, 12)
+    ref_e = oracle.paged_attention(qe, e.k_log, e.v_log, e.table, e.ctx, SCALE, nthreads=16)
     first = run_decode(a, qa, torch.float32)
     check(first, run_decode(a, qa, torch.bfloat16), ref_a)
     for _ in range(3):
+        check(run_decode(e, qe, torch.float32), run_decode(e, qe, torch.bfloat16), ref_e)
         check(run_decode(b, qb, torch.float32), run_decode(b, qb, torch.bfloat16), ref_b)
         check(run_decode(c, qc, torch.float32), run_decode(c, qc, torch.bfloat16), ref_c)
         assert np.array_equal(run_decode(a, qa, torch.float32), first)

@@ -28,7 +28,8 @@ def _run(case, q_bits, out_dtype, no_alloc):
 
 def test_no_alloc_matches_paged_attention_on_two_calls():
     big = make_case(71, oracle.randint(16, 64, 512, 8192).astype(np.int32))
-    small = make_case(73, oracle.randint(17, 9, 1, 700).astype(np.int32))
+    # (a table too wide for the one workgroup per unit: split records again)
+    small = make_case(73, oracle.randint(17, 9, 1, 700).astype(np.int32), extra_pages=60)
     for name, case, seed in (("B=64 ctx U[512,8192]", big, 72), ("B=9 ctx U[1,700]", small, 74)):
         print(f"[no_alloc] {name}", flush=True)
         q = queries(seed, case.B, 12)
