@@ -139,8 +139,8 @@ __device__ bool blockGeom(const Args &a, int b, int block, int pps, TileGeom &t,
 // the output's own, and it halves the record bytes that the attention kernel
 // writes and the combine reads. fp32 outputs keep fp32 records. The (m, l)
 // pairs stay fp32 after the O block either way.
-// (Chosen splits, of batches that would have had one or few, keep fp32
-// records too.)
+// (Splits finer than a.pps, of batches that would have had one or few, keep
+// fp32 records too.)
 template <bool OUT_F32> __device__ __forceinline__ void storeRecordO(float *rec, int idx, f32x4 v) {
     if constexpr (OUT_F32) {
         *reinterpret_cast<f32x4 *>(rec + idx) = v;
@@ -362,7 +362,13 @@ __device__ __forceinline__ void prefillItem(const Args &a, StageBuf &kvs, int b,
         }
         const int c = k * 16 + n; // column within the group
 #pragma unroll
-        for (int i = 0; i < 8; ++i) storeRecordO<OUT_F32 || CHOOSE>(rec, (i * kTiles * 16 + c) * 16 + grp * 4, acc[k].o[i]);
+        for (int i = 0; i < 8; ++i) {
+            const int at = (i * kTiles * 16 + c) * 16 + grp * 4;
+            if (CHOOSE && pps < a.pps)
+                storeRecordO<true>(rec, at, acc[k].o[i]);
+            else
+                storeRecordO<OUT_F32>(rec, at, acc[k].o[i]);
+        }
         if (grp == 0)
             *reinterpret_cast<float2 *>(rec + kTiles * 16 * kHeadDim + 2 * c) = make_float2(acc[k].m, lt);
     }
@@ -615,7 +621,7 @@ __global__ void __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_e
     // 64 per register; wave w ranks sequences w, w + kWaves, ..., a ballot
     // per register counting those ahead (a loop over the batch in LDS per
     // thread was 2 us of LDS latency at B = 64).
-    int n_dec_seqs = 0;
+    int n_dec_seqs = 0, dec_pages = 0;
     if constexpr (WITH_DECODE) {
         constexpr int kRegs = kQueueSortSeqs / 64;
         const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
@@ -625,7 +631,9 @@ __global__ void __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_e
             const int o = 64 * r + lane;
             ko[r] = o < B ? dkey[o] : -1;
             n_dec_seqs += __popcll(__ballot(ko[r] >= 0));
+            if constexpr (CHOOSE) dec_pages += ko[r] >= 0 ? (ko[r] + 15) >> 4 : 0;
         }
+        if constexpr (CHOOSE) dec_pages = __builtin_amdgcn_readlane(waveInclusiveSum(dec_pages), 63);
         for (int b = wave; b < B; b += kWaves) {
             int kb = ko[0];
 #pragma unroll
@@ -669,22 +677,32 @@ __global__ void __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_e
             setSplits(u, np, a.pps);
     }
     __syncthreads();
-    // Pages per split: the fewest (a multiple of a stage, from pps_min) whose
-    // items still fit the CUs in one round, else pps. A split of 64 pages
-    // takes 45 us however few of them there are; finer ones than one round
-    // only add records (us with 64 pages / chosen, 12:2 heads: one prompt of
-    // 1000 tokens 44.5 / 34.6, of 2000 52.3 / 47.0, prompts of 350, 650 and
-    // 950 43.5 / 38.1, 64 tokens after 1000 46.2 / 27.9, 512 after 1500 48.0 /
-    // 38.0, six chunks of 100 after 2000 49.0 / 39.8).
-    // Every wave works it out by itself, from the coarsest down.
+    // Pages per split: as few (a multiple of a stage, from pps_min) as leave
+    // every CU one item at most, the single-query sequences' among them, and
+    // no fewer than take as long as those do (a page of a split 0.7 us; of the
+    // longest context 0.07 us, and all their pages' heads 1.6 ns of HBM each):
+    // finer splits would only add records to merge. Else pps. A split of 64
+    // pages takes 45 us however few of them there are (us with 64 pages /
+    // chosen, 12:2 heads: one prompt of 600 tokens 31.8 / 26.4, of 1000 43.3 /
+    // 32.0, of 2000 50.4 / 46.6, two of 1200 49.8 / 42.3, 64 tokens after 2000
+    // 46.0 / 27.4, 512 after 1500 47.1 / 35.4, after 4000 52.4 / 44.7).
+    // Every wave works it out by itself.
     int pps = a.pps;
     if constexpr (CHOOSE) {
-        for (int cand = pps - 2 * kStagePairs; cand >= a.pps_min; cand -= 2 * kStagePairs) {
-            const float inv = 1.f / float(cand);
-            int items = 0; // (rounding here moves a choice, not a result)
-            for (int u = tid & 63; u < U; u += 64) items += int(float(nspl[u] + cand - 1) * inv);
-            if (__builtin_amdgcn_readlane(waveInclusiveSum(items), 63) > a.cus) break;
-            pps = cand;
+        int pages = 0;
+        for (int u = tid & 63; u < U; u += 64) pages += nspl[u];
+        pages = __builtin_amdgcn_readlane(waveInclusiveSum(pages), 63);
+        const int free = a.cus - n_dec - U;
+        if (free > 0) {
+            float want = float(pages) * __builtin_amdgcn_rcpf(float(free)); // (rounding moves a choice, not a result)
+            if (n_dec_seqs > 0) {
+                const float longest = float(ctx[dseq[0]]) * (1.f / 16.f);
+                want = fmaxf(want, fmaxf(0.1f * longest, 0.0023f * float(dec_pages * a.nkvh)));
+            }
+            constexpr int kStep = 2 * kStagePairs;
+            const int fewest = __builtin_amdgcn_readfirstlane(int(fminf(want, 1024.f))); // a scalar, as loop bounds
+            const int cand = max(a.pps_min, (fewest + kStep - 1) & ~(kStep - 1));
+            if (4 * cand <= 3 * pps) pps = cand;
         }
         __syncthreads(); // every wave has read the page counts, which the splits replace
         for (int u = tid; u <= U; u += nthreads) setSplits(u, nspl[u], pps);
@@ -782,31 +800,38 @@ template <bool OUT_F32, bool CHOOSE> __global__ void __launch_bounds__(64) prefi
     f32x4 o[8];
 #pragma unroll
     for (int i = 0; i < 8; ++i) o[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-    for (int k0 = 0; k0 < t.nsplit; k0 += kMergeBatch) {
-        float mr[kMergeBatch], lr[kMergeBatch];
-        f32x4 orr[kMergeBatch][8];
+    auto merge = [&](auto f32) {
+        constexpr bool RECORDS_F32 = decltype(f32)::value;
+        for (int k0 = 0; k0 < t.nsplit; k0 += kMergeBatch) {
+            float mr[kMergeBatch], lr[kMergeBatch];
+            f32x4 orr[kMergeBatch][8];
 #pragma unroll
-        for (int s = 0; s < kMergeBatch; ++s) {
-            const float *rec = recs + size_t(min(k0 + s, t.nsplit - 1)) * kRecordFloats;
-            const float2 ml = *reinterpret_cast<const float2 *>(rec + kTiles * 16 * kHeadDim + 2 * c);
-            mr[s] = k0 + s < t.nsplit ? ml.x : -INFINITY;
-            lr[s] = ml.y;
+            for (int s = 0; s < kMergeBatch; ++s) {
+                const float *rec = recs + size_t(min(k0 + s, t.nsplit - 1)) * kRecordFloats;
+                const float2 ml = *reinterpret_cast<const float2 *>(rec + kTiles * 16 * kHeadDim + 2 * c);
+                mr[s] = k0 + s < t.nsplit ? ml.x : -INFINITY;
+                lr[s] = ml.y;
 #pragma unroll
-            for (int i = 0; i < 8; ++i) orr[s][i] = loadRecordO<OUT_F32 || CHOOSE>(rec, (i * kTiles * 16 + c) * 16 + grp * 4);
+                for (int i = 0; i < 8; ++i) orr[s][i] = loadRecordO<RECORDS_F32>(rec, (i * kTiles * 16 + c) * 16 + grp * 4);
+            }
+#pragma unroll
+            for (int s = 0; s < kMergeBatch; ++s) {
+                // A split can lie wholly past a column's causal limit: m = -inf, weight 0.
+                if (mr[s] == -INFINITY) continue;
+                const float Mn = fmaxf(M, mr[s]);
+                const float sa = exp2Fast(M - Mn);
+                const float sb = exp2Fast(mr[s] - Mn);
+                L = L * sa + lr[s] * sb;
+#pragma unroll
+                for (int i = 0; i < 8; ++i) o[i] = o[i] * sa + orr[s][i] * sb;
+                M = Mn;
+            }
         }
-#pragma unroll
-        for (int s = 0; s < kMergeBatch; ++s) {
-            // A split can lie wholly past a column's causal limit: m = -inf, weight 0.
-            if (mr[s] == -INFINITY) continue;
-            const float Mn = fmaxf(M, mr[s]);
-            const float sa = exp2Fast(M - Mn);
-            const float sb = exp2Fast(mr[s] - Mn);
-            L = L * sa + lr[s] * sb;
-#pragma unroll
-            for (int i = 0; i < 8; ++i) o[i] = o[i] * sa + orr[s][i] * sb;
-            M = Mn;
-        }
-    }
+    };
+    if (CHOOSE && pps < a.pps)
+        merge(std::true_type());
+    else
+        merge(std::bool_constant<OUT_F32>());
     if (!col_ok) return;
     const float inv = 1.f / L;
     const size_t row = (size_t(t.q0 + qi) * a.nh + h * G + g) * kHeadDim;
@@ -837,6 +862,12 @@ int cuCount() {
 
 } // namespace
 
+// Whether the persistent kernel's item tables fit in LDS beside the stages.
+static bool queueFits(int B, const PagedAttentionPlan &plan) {
+    return envInt("LLAISYS_PREFILL_QUEUE", 1) != 0 && B <= kQueueMaxSeqs && plan.block_units <= kQueueMaxUnits &&
+           queueTableInts(B, plan.block_units) * sizeof(int) <= kQueueTableBytes;
+}
+
 PagedAttentionPlan planPrefill(int B, int T, int nkvh, int group, int max_pages) {
     PagedAttentionPlan p{};
     const int groups = ((T * group + 15) / 16 + kTiles - 1) / kTiles + B; // upper bound over the batch
@@ -850,15 +881,26 @@ PagedAttentionPlan planPrefill(int B, int T, int nkvh, int group, int max_pages)
     p.pages_per_split = pps;
     // Batches whose blocks of queries leave CUs idle may take finer splits
     // (down to 16 pages, chosen on the device, which knows the lengths), as
-    // far as 256 MiB of records go. Not where tables full of 64-page splits
-    // would give every CU one and a half: the choice is 64 there, and reading
-    // it back costs the merge a microsecond (the benchmark's mixed step 94.4
-    // us fixed, 95.6 chosen). Tables of up to 32 pages keep one split and no
-    // merge: at most 8 stages of a split, and the merge costs two.
+    // far as 256 MiB of records go: one sequence, or so many queries that few
+    // sequences can be single ones. Beside decodes the choice mostly cost more
+    // than it gave (us, fixed / chosen: 200 tokens and a decode of 4000 28.5 /
+    // 33.2, two chunks of 256 and 60 decodes to 4000 59.6 / 63.8). Not where
+    // tables full of 64-page splits would give three quarters of the CUs an
+    // item: the choice is 64 there for most lengths, and reading it back costs
+    // the merge a microsecond (2048 after 2000 91 / 98; a short prompt alone in
+    // a wide table 16.2 / 17.5). Tables of up to 64 pages need no merge
+    // otherwise, whose launch costs 5 us: only where the queries show that the
+    // contexts are long (a prompt of 600 tokens 31.8 / 26.4, of 1000 43.3 /
+    // 32.0, three of 350, 650 and 950 42.7 / 34.8) and, of several, that one
+    // may be much longer than the average (three of 700 35.0 / 34.9; but in 34
+    // pages four of 530 29.2 / 33.3).
     p.pages_per_split_min = pps;
+    p.max_splits = std::max(1, (max_pages + pps - 1) / pps);
     const long long blocks = ((long long)T * group + kWaves * kTiles * 16 - 1) / (kWaves * kTiles * 16) * nkvh;
-    if (!std::getenv("LLAISYS_PAGES_PER_SPLIT") && max_pages > 32 && blocks < cuCount() &&
-        blocks * max_pages < 96LL * cuCount()) {
+    const bool long_ones = T >= 512LL * B;
+    const bool pays = max_pages > 64 ? (B == 1 || long_ones) && blocks * max_pages < 48LL * cuCount()
+                                     : long_ones && 2 * blocks <= cuCount() && (B == 1 || max_pages > 40);
+    if (!std::getenv("LLAISYS_PAGES_PER_SPLIT") && pays && blocks < cuCount() && queueFits(B, p)) {
         constexpr size_t kMostBytes = size_t(256) << 20;
         int least = 16;
         while (least < pps && size_t(p.units) * ((max_pages + least - 1) / least) * kRecordFloats * sizeof(float) > kMostBytes)
@@ -871,9 +913,7 @@ PagedAttentionPlan planPrefill(int B, int T, int nkvh, int group, int max_pages)
 }
 
 bool prefillQueueUsable(int B, const PagedAttentionPlan &plan, const int *queue) {
-    return queue && envInt("LLAISYS_PREFILL_QUEUE", 1) != 0 && B <= kQueueMaxSeqs &&
-           plan.block_units <= kQueueMaxUnits &&
-           queueTableInts(B, plan.block_units) * sizeof(int) <= kQueueTableBytes;
+    return queue && queueFits(B, plan);
 }
 
 bool prefillTakesDecode(int B, int T, const PagedAttentionPlan &plan, const int *queue) {
@@ -910,22 +950,22 @@ void pagedPrefill(void *out, bool out_f32, const uint16_t *q, const uint16_t *k_
     a.max_pages = max_pages;
     a.num_blocks = num_blocks;
     a.pps = plan.pages_per_split;
-    a.max_splits = plan.max_splits;
+    const bool queued = prefillQueueUsable(B, plan, queue);
+    a.pps_min = queued ? plan.pages_per_split_min : plan.pages_per_split;
+    a.max_splits = std::max(1, (max_pages + a.pps_min - 1) / a.pps_min);
     a.units = plan.units;
     a.block_units = plan.block_units;
     a.block_units_padded = plan.block_units_padded;
     a.scale_log2 = scale * 1.4426950408889634f;
-    const dim3 grid(plan.block_units_padded * plan.max_splits), block(64 * kWaves), cblock(64);
+    const dim3 grid(plan.block_units_padded * a.max_splits), block(64 * kWaves), cblock(64);
     auto s = static_cast<hipStream_t>(stream);
     // The persistent kernel whenever its item tables fit in LDS beside the
     // stages (and a counter buffer is given); otherwise one workgroup per
     // grid slot.
     const size_t table_bytes = queueTableInts(B, plan.block_units) * sizeof(int);
-    const bool queued = prefillQueueUsable(B, plan, queue);
     a.with_decode = queued && prefillTakesDecode(B, T, plan, queue);
-    a.pps_min = queued ? plan.pages_per_split_min : plan.pages_per_split;
     a.cus = cuCount();
-    const dim3 qgrid(unsigned(std::min<long long>(cuCount(), (long long)plan.block_units * plan.max_splits)));
+    const dim3 qgrid(unsigned(std::min<long long>(cuCount(), (long long)plan.block_units * a.max_splits)));
     const bool choose = a.pps_min < a.pps;
     auto launch = [&](auto f32, auto chosen) {
         constexpr bool F32 = decltype(f32)::value, CHOOSE = decltype(chosen)::value;
@@ -935,7 +975,7 @@ void pagedPrefill(void *out, bool out_f32, const uint16_t *q, const uint16_t *k_
             hipLaunchKernelGGL((prefillQueueKernel<F32, false, CHOOSE>), qgrid, block, unsigned(table_bytes), s, a);
         else
             hipLaunchKernelGGL((prefillKernel<F32>), grid, block, 0, s, a);
-        if (plan.max_splits > 1)
+        if (a.max_splits > 1)
             hipLaunchKernelGGL((prefillCombineKernel<F32, CHOOSE>), dim3(plan.units * kTiles), cblock, 0, s, a);
     };
     if (out_f32) {
