@@ -91,8 +91,9 @@ public:
     // One int32 of kernel-side error bits (device memory on AMD; on CPU a host
     // word the host ops raise bits in, read and cleared the same way).
     int *errorWord();
-    // Two int32 work-queue counters for persistent kernels, zeroed once; the
-    // kernels return them to zero before they end.
+    // kernels::kPrefillQueueWords int32 words for the persistent prefill kernel,
+    // zeroed once: two work-queue counters, which it returns to zero before it
+    // ends, and last the split size of its latest call, for that call's merge.
     int *queueCounters();
     // Bits raised since the last call (llaisysGetDeviceErrorFlags), then zero.
     int takeErrorFlags();

@@ -202,10 +202,11 @@ template <int BM, int BN, int NW> constexpr int wideStages() {
 // (~62 at ~290 cycles each) then bound the k loop. With 128 B per row a
 // block of one instruction is 8 rows x 128 B, piece c of row r sits at slot
 // c ^ (r % 8) (the 8 lanes one LDS cycle serves read 8 rows of one piece:
-// 8 distinct slots), and a stage is twice the bytes, so the ring holds two
-// stages: the next stage's loads go out right after the barrier that frees
-// its slot and have the current stage's two MFMA steps to land; the second
-// step's fragments are read under the first step's MFMAs.
+// 8 distinct slots), and a stage is twice the bytes, so the ring holds two to
+// four (wideStages): a stage's loads go out between the fragment reads after
+// the barrier that frees its slot, and have the MFMA steps of the stages
+// before it to land; the second step's fragments are read under the first
+// step's MFMAs.
 // WGM x WGN waves, wave (wm, wn) owning the (BM / WGM) x (BN / WGN) sub-tile.
 template <ElemType T, int BM, int BN, int WGM = 2, int WGN = 2, bool PIPE = false, int RB = 64, int WS = 2>
 __global__ void __launch_bounds__(64 * WGM * WGN) gemmKernel(GemmParams p) {

@@ -71,14 +71,15 @@ void pagedDecodeUnits(void *out, bool out_f32, const uint16_t *q, const uint16_t
                       int num_blocks, float scale, int *err, void *stream, uint16_t *out_packed = nullptr,
                       bool keep_invalid = false);
 // Whether a batch of contexts of up to max_pages pages takes it whatever their
-// spread: one launch instead of two while a unit is short (us, this /
-// stream-K, 12:2 heads): 1 x 300 tokens 5.9 / 8.6, 1 x 700 9.0 / 10.1, 64 x
-// 50-200 5.9 / 9.5, 128 x 64-448 9.2 / 14.2. Past the line a call waits for
-// the one CU of a unit (55 GB/s): 1 x 1500 16.2 / 11.0; with 128 units and
-// more every CU has one, and it lies further out: 64 x 300-800 11.6 / 13.8, 64
-// x 1000-2000 23.6 / 23.6.
+// spread (the host knows the table's width, not the lengths): one launch
+// instead of two while a unit is short (us, this / stream-K in a wider table,
+// 12:2 heads): 1 x 300 tokens 6.3 / 8.4, 1 x 700 9.7 / 9.9, 64 x 50-200 5.5 /
+// 9.4, 128 x 64-448 8.0 / 13.5. Past the line a call waits for the one CU of a
+// unit (55 GB/s): 1 x 768 10.2 / 9.6; with 128 units and more every CU has
+// one, and it lies further out: 64 x 300-800 11.3 / 13.4, 64 x 600-1024 13.2 /
+// 15.3.
 inline bool unitDecodeTakes(int B, int nkvh, int max_pages) {
-    return max_pages <= ((long long)B * nkvh >= 128 ? 64 : 48);
+    return max_pages <= ((long long)B * nkvh >= 128 ? 64 : 44);
 }
 
 // pagedDecodeUnits with the decode step's QKV epilogue fused in (one token per

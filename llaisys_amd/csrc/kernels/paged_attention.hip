@@ -12,7 +12,8 @@
 // Query qi of a sequence with Lq new tokens sits at position ctx - Lq + qi
 // and sees keys at positions <= that (bottom-right causal alignment). A
 // block's visible pages (up to its last query) are cut into splits of
-// `pages_per_split` pages; one workgroup runs one (block, split): the next
+// `pages_per_split` pages, or of fewer where the persistent kernel below may
+// choose (planPrefill); one workgroup runs one (block, split): the next
 // pair is loaded into registers while the current one is consumed from LDS
 // (loads never conditional: past the end they re-read the last pair), into
 // the MFMA step of mfma_common.hpp. A unit with one split writes its normalised

@@ -3,9 +3,9 @@
 // Work = every (sequence b, kv head h) unit's page pairs, laid end to end:
 // unit u = b*nkvh + h owns npairs(b) = ceil(ceil(ctx_b/16)/2) consecutive
 // pair indices. A grid of W single-wave workgroups (about one per CU) splits
-// the N pairs evenly: wave w takes pairs [w*P, (w+1)*P), P = ceil(N/W) <= 64
-// (the last waves take what is left), and
-// streams them through a ring of NSTAGE page pairs in flight, crossing unit
+// the N pairs evenly: wave w takes pairs [w*P, (w+1)*P), P <= 64 (the last
+// waves take what is left): ceil(N/W), or more where that would cut few long
+// units finer than their records pay for (pairsPerWave). It streams them through a ring of NSTAGE page pairs in flight, crossing unit
 // boundaries without draining the ring. Every wave does the same small prefix
 // scan of ctx into LDS to find its slice, so no host-side knowledge of the
 // lengths and no planning kernel is needed.
@@ -16,13 +16,12 @@
 // launched next on the same stream, merges each split unit's records with
 // log-sum-exp weights. A unit spread over at most `slots` waves keeps its
 // records in slots of its own (slot k = the wave's place among the unit's
-// waves) in a persistent buffer, each with a header holding the record count:
-// the combine then finds them without knowing the lengths, in one memory
-// round trip, and returns the headers to zero. A unit spread further uses
-// per-wave records (slot 0:
-// the wave's first unit, slot 1: its last) with slot 0's header set to -1, and
-// the combine locates them through the length scan. The kernel boundary makes the records visible to the
-// combine on every XCD. (Merging inside this kernel instead needs either
+// waves) in a persistent buffer, slot 0 with a header holding the record count:
+// the combine then finds them without knowing the lengths, the first 8 in one
+// memory round trip, and returns the header to zero. A unit spread further uses
+// per-wave records (record 0: the wave's first unit, 1: its last) with its
+// header set to -1, and the combine locates them through the length scan. The
+// kernel boundary makes the records visible to the combine on every XCD. (Merging inside this kernel instead needs either
 // agent-scope fences, which write back / invalidate a whole L2 per wave, or
 // device-scope record traffic plus a serial merge at the tail; both measured
 // slower than the second launch.)
