@@ -114,8 +114,7 @@ template <int PARTS> struct PairP {
 // Parts of the decode kernels' weights: one would show beside a bf16 result's
 // own rounding, two beside a 32-bit result's (2-norm of the error, 700 tokens:
 // 2.3e-3 -> 1.66e-3 and 2.3e-6 -> 2.5e-7 with the second and third part; 9.0 ->
-// 10.0 and 9.8 -> 10.9 us, and nothing where HBM is the bound: 64 x 512-8192
-// 52.1 -> 52.3).
+// 10.0 and 9.8 -> 10.9 us).
 template <bool OUT_F32> constexpr int decodeParts() { return OUT_F32 ? 3 : 2; }
 
 // Raw scores of one page pair (K pages a, b) against the lane's column of

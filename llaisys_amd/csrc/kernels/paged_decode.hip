@@ -39,6 +39,7 @@
 #include <cstddef>
 #include <cstdlib>
 #include <mutex>
+#include <type_traits>
 #include <vector>
 
 namespace llaisys::kernels {
@@ -54,6 +55,11 @@ constexpr int kMergeBatch = 4;    // records whose loads are in flight together
 // are cut into many pieces; kFirstSlots, which the combine requests before it
 // knows how many are used, for larger ones.
 constexpr int kFirstSlots = 8, kManySlots = 32, kManySlotUnits = 512;
+// Batches of up to this many units take slices of a least size (pairsPerWave)
+// and their weights in one more part, which the longer records need; larger
+// ones, whose even slices are longer anyway, stream at the memory's rate, where
+// the part shows (64 x 512-8192 53.4 us without, 54.1 with).
+constexpr int kFewUnits = 64;
 
 struct DecodeArgs {
     const uint16_t *q;
@@ -71,6 +77,7 @@ struct DecodeArgs {
     uint16_t *out_packed; // non-null (bf16 out): rows go there in operand order (packedRowIndex) instead of to out
     int B, T, nh, nkvh, G, max_pages, num_blocks, W;
     int slots; // record slots per unit
+    int few;   // at most kFewUnits units
     float scale_log2;
 };
 
@@ -145,11 +152,11 @@ __device__ int scanPairs(const DecodeArgs &a, int *S, int *C, int *Q, bool repor
 // 3 pairs a wave (0.3 us each) avoid it. A few long sequences over all the
 // waves left a record per page pair, and merging them took longer than the
 // stream; one sequence of 1500 / 4000 / 16000 tokens, 12:2 heads: 15.7 / 27.1
-// / 35.3 us without this rule, 11.0 / 13.0 / 21.6 with it. Larger batches
-// (kFirstSlots) leave the few units that are cut finer to the per-wave records.
+// / 35.3 us without this rule, 11.5 / 13.6 / 23.1 with it. Larger batches
+// (past kFewUnits) leave the few units that are cut finer to the per-wave records.
 __device__ __forceinline__ int pairsPerWave(const DecodeArgs &a, int N, int longest) {
     int least = 1;
-    if (a.slots != kFirstSlots)
+    if (a.few)
         least = max(min(kPairsPerWave, (longest + kManySlots - 2) / (kManySlots - 1)),
                     min(3, (longest + kFirstSlots - 2) / (kFirstSlots - 1)));
     return max((N + a.W - 1) / a.W, least);
@@ -176,7 +183,7 @@ template <int NSTAGE> struct Ring {
 // register file (one wave per SIMD) to avoid spilling. PACKED (bf16): rows
 // go to a.out_packed; a separate instance, since the branch in the finish
 // cost the plain kernel 14 % (53.8 -> 61.3 us at config 3).
-template <bool OUT_F32, int NSTAGE, bool PACKED = false>
+template <bool OUT_F32, int NSTAGE, bool FEW, bool PACKED = false>
 __global__ void __launch_bounds__(64)
     __attribute__((amdgpu_waves_per_eu(NSTAGE == 2 ? 2 : 1, NSTAGE == 2 ? 2 : 1))) decodeKernel(DecodeArgs a) {
     extern __shared__ int lds[];
@@ -346,7 +353,7 @@ __global__ void __launch_bounds__(64)
                 u32x4 qop[4];
 #pragma unroll
                 for (int t = 0; t < 4; ++t) qop[t] = n < G ? ring.q[st][t] : u32x4{0, 0, 0, 0};
-                consumePair<decodeParts<OUT_F32>()>(acc, ring.pp[st], qop, 32 * j, c - 1, c, hasB, grp, a.scale_log2);
+                consumePair<decodeParts<OUT_F32>() - (FEW ? 0 : 1)>(acc, ring.pp[st], qop, 32 * j, c - 1, c, hasB, grp, a.scale_log2);
             }
             issue(st, k + NSTAGE);
         }
@@ -999,6 +1006,7 @@ void pagedDecode(void *out, bool out_f32, const uint16_t *q, const uint16_t *k_p
     a.slot_hdr = slots ? slot_headers : nullptr;
     a.slot_rec = slots ? static_cast<float *>(slot_records) : nullptr;
     a.slots = slotsFor(B, nkvh);
+    a.few = (long long)B * nkvh <= kFewUnits;
     a.B = B;
     a.T = T;
     a.nh = nh;
@@ -1011,27 +1019,22 @@ void pagedDecode(void *out, bool out_f32, const uint16_t *q, const uint16_t *k_p
     auto s = static_cast<hipStream_t>(stream);
     const unsigned lds = unsigned(plan.lds_bytes);
     const dim3 grid(plan.waves), block(64), comb(B * nkvh), comb_block(64 * kCombineWaves);
-    if (out_f32) {
+    auto launch = [&](auto f32, auto few, auto packed) {
+        constexpr bool F32 = decltype(f32)::value, FEW = decltype(few)::value, PACKED = decltype(packed)::value;
         if (plan.stages == 3)
-            hipLaunchKernelGGL((decodeKernel<true, 3>), grid, block, lds, s, a);
+            hipLaunchKernelGGL((decodeKernel<F32, 3, FEW, PACKED>), grid, block, lds, s, a);
         else
-            hipLaunchKernelGGL((decodeKernel<true, 2>), grid, block, lds, s, a);
-        hipLaunchKernelGGL((decodeCombineKernel<true>), comb, comb_block, lds, s, a);
-    } else {
-        if (out_packed) {
-            if (plan.stages == 3)
-                hipLaunchKernelGGL((decodeKernel<false, 3, true>), grid, block, lds, s, a);
-            else
-                hipLaunchKernelGGL((decodeKernel<false, 2, true>), grid, block, lds, s, a);
-            hipLaunchKernelGGL((decodeCombineKernel<false, true>), comb, comb_block, lds, s, a);
-        } else {
-            if (plan.stages == 3)
-                hipLaunchKernelGGL((decodeKernel<false, 3>), grid, block, lds, s, a);
-            else
-                hipLaunchKernelGGL((decodeKernel<false, 2>), grid, block, lds, s, a);
-            hipLaunchKernelGGL((decodeCombineKernel<false>), comb, comb_block, lds, s, a);
-        }
-    }
+            hipLaunchKernelGGL((decodeKernel<F32, 2, FEW, PACKED>), grid, block, lds, s, a);
+        hipLaunchKernelGGL((decodeCombineKernel<F32, PACKED>), comb, comb_block, lds, s, a);
+    };
+    const std::true_type yes;
+    const std::false_type no;
+    if (out_f32)
+        a.few ? launch(yes, yes, no) : launch(yes, no, no);
+    else if (out_packed)
+        a.few ? launch(no, yes, yes) : launch(no, no, yes);
+    else
+        a.few ? launch(no, yes, no) : launch(no, no, no);
     HIP_CHECK(hipGetLastError());
 }
 
