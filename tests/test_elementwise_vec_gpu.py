@@ -39,7 +39,10 @@ def test_add_and_swiglu(n, off, dtype):
 @pytest.mark.parametrize("dtype", list(TYPES))
 @pytest.mark.parametrize("rows,d", [(1, 1), (3, 7), (5, 8), (2, 520), (9, 1536), (4, 2048), (3, 2052), (2, 4096),
                                     (2, 4104), (1, 10000), (1025, 8), (1027, 7),
-                                    (1026, 520), (1030, 1536), (1025, 2052), (1026, 4096), (1025, 4104)])
+                                    (1026, 520), (1030, 1536), (1025, 2052), (1026, 4096), (1025, 4104),
+                                    # a wave per row from 2049 rows, long rows from 3073
+                                    (2048, 8), (2049, 8), (2050, 520), (2051, 1536), (2049, 1024), (3072, 4096),
+                                    (3073, 2052), (3074, 4096), (3073, 4104)])
 @pytest.mark.parametrize("off", [0, 1])
 def test_rms_norm(rows, d, off, dtype):
     x, w = rnd((rows, d), dtype, 3), rnd((d,), dtype, 4)
@@ -52,7 +55,9 @@ def test_rms_norm(rows, d, off, dtype):
 
 
 @pytest.mark.parametrize("dtype", list(TYPES))
-@pytest.mark.parametrize("tokens,heads,d", [(1, 1, 2), (3, 5, 12), (7, 12, 128), (2, 40, 64), (2, 1, 1024), (2, 2, 1040)])
+@pytest.mark.parametrize("tokens,heads,d", [(1, 1, 2), (3, 5, 12), (7, 12, 128), (2, 40, 64), (2, 1, 1024), (2, 2, 1040),
+                                            # around a wave of elements, and shared angles with ragged halves
+                                            (4, 2, 64), (4, 2, 80), (3, 3, 44), (7, 12, 36), (2, 2, 1024), (3, 1, 128)])
 @pytest.mark.parametrize("off", [0, 1])
 def test_rope(tokens, heads, d, off, dtype):
     x = rnd((tokens, heads, d), dtype, 5)
